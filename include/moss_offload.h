@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define MO_ABI_VERSION 21
+#define MO_ABI_VERSION 22
 #define MO_MAX_DIMS 8
 
 /* Error codes outside the hipError_t range. */
@@ -506,6 +506,27 @@ int mo_int8_set_kernel(uint32_t kernel);
  * library's launches, for tests and tools. */
 int mo_int8_launch_plan(uint32_t rows, uint32_t cols, uint32_t reduction, uint32_t cus, uint32_t kernel,
                         uint32_t* n_parts, uint32_t* parts);
+
+/* The same two products on the strip kernels, for calls with few rows: five tile shapes, the
+ * reduction shared out inside a workgroup and over workgroups as a cost model picks, the weight
+ * read as it is stored in both directions (no transposed copy). Same operands and constraints as
+ * mo_int8_linear_forward / backward, and the reduction (in_features, out_features for the input
+ * gradient) a multiple of 64. One kernel launch, two where the plan splits the reduction over
+ * workgroups; then `workspace` (device, 16-byte aligned, at least mo_int8_strip_workspace_bytes(rows,
+ * cols, reduction) bytes) holds the fp32 partial sums. Without one (0) nothing is split. The same
+ * call gives the same bits every time. Replaces the reference's kernels as those above do. */
+int mo_int8_strip_forward(uint64_t x, uint64_t w, uint64_t scale, uint64_t bias, uint64_t y, uint32_t rows,
+                          uint32_t in_features, uint32_t out_features, uint64_t workspace, uint64_t workspace_bytes,
+                          uint64_t stream);
+int mo_int8_strip_backward(uint64_t dy, uint64_t w, uint64_t scale, uint64_t dx, uint32_t rows, uint32_t in_features,
+                           uint32_t out_features, uint64_t workspace, uint64_t workspace_bytes, uint64_t stream);
+uint64_t mo_int8_strip_workspace_bytes(uint32_t rows, uint32_t cols, uint32_t reduction);
+
+/* The strip plan of such a call on a device of `cus` CUs, host only: plan[0..4] = tile rows, tile
+ * columns, K groups of a workgroup, splits (workgroups per tile; 1 without may_split), steps of 64
+ * per split. For tests and tools. */
+int mo_int8_strip_plan(uint32_t rows, uint32_t cols, uint32_t reduction, uint32_t cus, uint32_t may_split,
+                       uint32_t* plan);
 
 /* ---- host gradient accumulation (training/fused_adafactor.py:327-369) -------------------- */
 

@@ -1,5 +1,6 @@
 // Host side of the int8 weight-only GEMMs (csrc/mo_gemm.hip): argument checks, module loading
-// from the embedded gfx950 code object, the launch plan. C ABI: mo_int8_linear_forward/backward.
+// from the embedded gfx950 code object, the launch plans. C ABI: mo_int8_linear_forward/backward
+// (the plan below) and mo_int8_strip_forward/backward (strip_plan, for calls with few rows).
 //
 // Launch plan: the large tile (256 x 256) carries the work; when its grid would leave the GPU's
 // last round of workgroups less than half full, the rows of that partial round go to a second
@@ -47,7 +48,29 @@ struct GemmModule {
   hipFunction_t ws_kscale = nullptr;  // mo_int8_ws_kscale: the same on a transposed weight, per-k scales
   hipFunction_t transpose = nullptr;  // mo_int8_transpose_kernel
   hipFunction_t ws_fwd_split = nullptr, ws_kscale_split = nullptr, split_reduce = nullptr;
+  hipFunction_t strip[2][5] = {};  // [backward][kStrips index]
 };
+
+// The strip kernels (mo_gemm.hip): output tile, K groups of a workgroup, and what the cost model
+// knows of them on an MI355X, in us: a call's fixed part, and a step of 64 of every K group with
+// one workgroup on a CU and with `resident` (all that fit). Fitted to 5 300 timed calls (64 to
+// 5 500 rows of ten weight shapes, both directions, one to 32 splits): the model's choice takes
+// 1.4 % longer than the fastest one on average, 18 % at worst.
+struct Strip {
+  const char* name;
+  uint32_t bm, bn, k_groups;
+  int resident;
+  double fixed, alone, together;
+};
+constexpr int kStripCount = 5;
+constexpr Strip kStrips[kStripCount] = {
+    {"128x256", 128, 256, 1, 2, 6.0, 0.73, 1.38},    // wide grids
+    {"128x256k2", 128, 256, 2, 1, 6.6, 1.40, 1.40},  // long reductions over few tiles
+    {"128x128", 128, 128, 1, 3, 4.6, 0.55, 1.22},    // grids between one and two rounds
+    {"64x64k4", 64, 64, 4, 1, 6.3, 0.67, 0.67},      // a 3 072-wide output of a few hundred rows
+    {"32x64k4", 32, 64, 4, 2, 4.0, 0.49, 1.31},      // fewer rows than that
+};
+constexpr double kStripReduce = 1.5, kStripReducePerMb = 0.28;  // the plane sum: fixed, per MB of planes
 
 // Which kernel takes the large-tile rows of a launch plan (mo_int8_set_kernel).
 std::atomic<uint32_t> g_kernel{MO_INT8_KERNEL_REGISTERS};
@@ -87,6 +110,12 @@ int gemm_module(GemmModule* out) {
         (e = hipModuleGetFunction(&m.ws_kscale_split, m.module, "mo_int8_ws_kscale_split")) != hipSuccess ||
         (e = hipModuleGetFunction(&m.split_reduce, m.module, "mo_int8_split_reduce")) != hipSuccess)
       return mo::set_hip_error((int)e, "hipModuleGetFunction (int8 weight-in-registers kernels)");
+    for (int bwd = 0; bwd < 2; ++bwd)
+      for (int i = 0; i < kStripCount; ++i) {
+        const std::string name = std::string("mo_int8_strip_") + (bwd ? "bwd_" : "fwd_") + kStrips[i].name;
+        if ((e = hipModuleGetFunction(&m.strip[bwd][i], m.module, name.c_str())) != hipSuccess)
+          return mo::set_hip_error((int)e, "hipModuleGetFunction (int8 strip)");
+      }
     it = g_modules.emplace(device, m).first;
   }
   *out = it->second;
@@ -198,6 +227,20 @@ int launch(const Kernel& k, void** params, uint32_t rows, uint32_t cols, uint64_
 // The weight-in-registers kernels: 256 x 256 tiles, four waves.
 Kernel registers_kernel(hipFunction_t fn) { return Kernel{fn, 256, kLarge}; }
 
+// Sums a split launch's fp32 planes into C (rows x cols bf16; bias may be 0).
+int launch_split_reduce(const GemmModule& m, uint64_t planes, uint64_t bias, uint64_t c, uint32_t rows, uint32_t cols,
+                        uint32_t splits, uint64_t stream) {
+  const void* P = (const void*)planes;
+  const void* Bi = (const void*)bias;
+  void* C = (void*)c;
+  void* params[] = {&P, &Bi, &C, &rows, &cols, &splits};
+  const uint64_t lanes = (uint64_t)rows * (cols / 8);
+  const hipError_t e = hipModuleLaunchKernel(m.split_reduce, (uint32_t)((lanes + 255) / 256), 1, 1, 256, 1, 1, 0,
+                                             (hipStream_t)stream, params, nullptr);
+  if (e != hipSuccess) return mo::set_hip_error((int)e, "int8 split reduction launch");
+  return 0;
+}
+
 // A split part: `splits` x tiles workgroups of the split kernel writing fp32 planes to `planes`,
 // then the reduction into C (rows of the part, `cols` wide; bias may be 0).
 int launch_split(const GemmModule& m, hipFunction_t fn, const Part& part, uint64_t a, uint64_t b, uint64_t scale,
@@ -213,15 +256,91 @@ int launch_split(const GemmModule& m, hipFunction_t fn, const Part& part, uint64
   hipError_t e = hipModuleLaunchKernel(fn, (uint32_t)(tiles_m * tiles_c * part.splits), 1, 1, 256, 1, 1, 0,
                                        (hipStream_t)stream, params, nullptr);
   if (e != hipSuccess) return mo::set_hip_error((int)e, "int8 GEMM split launch");
-  const void* Pc = (const void*)planes;
+  return launch_split_reduce(m, planes, bias, c, part.rows, cols, part.splits, stream);
+}
+
+// A strip call: shape, workgroups per tile and the reduction steps of 64 each covers.
+struct StripPlan {
+  int shape;
+  uint32_t splits, split_steps;
+};
+
+uint64_t div_up(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
+
+// Modelled time (us) of a strip call with `splits` workgroups per tile, of `per` steps each.
+double strip_cost(const Strip& s, uint32_t rows, uint32_t cols, uint32_t splits, uint32_t per, int cus) {
+  const uint64_t each = div_up(div_up(rows, s.bm) * div_up(cols, s.bn) * splits, (uint64_t)cus);  // workgroups a CU
+  const uint64_t rounds = each / s.resident, left = each % s.resident;
+  const uint64_t steps = (div_up(per, s.k_groups) + 1) & ~1ull;  // the loop runs steps in pairs
+  double step = (double)rounds * s.together;
+  if (left) step += s.alone + (s.together - s.alone) * (double)(left - 1) / (s.resident > 1 ? s.resident - 1 : 1);
+  double cost = s.fixed + (double)steps * step;
+  if (splits > 1) cost += kStripReduce + kStripReducePerMb * (double)splits * rows * cols * 4e-6;
+  return cost;
+}
+
+// The cheapest strip call. Splits: at most 32, of at least 6 steps (64-row tiles of four K groups
+// at least 8, two a group), while the workgroups stay within four and a half rounds of the CUs (more only pay for
+// planes). The 64 x 64 tile, one workgroup a CU, only while its grid fits one round: past it the
+// 32-row tile, two a CU, or the 128-row ones were faster at every size measured.
+StripPlan strip_plan(uint32_t rows, uint32_t cols, uint32_t steps, int cus, bool may_split) {
+  StripPlan best{0, 1, steps};
+  double best_cost = 0;
+  for (int i = 0; i < kStripCount; ++i) {
+    const Strip& s = kStrips[i];
+    const uint64_t tiles = div_up(rows, s.bm) * div_up(cols, s.bn);
+    uint32_t tried = 0;
+    for (uint32_t want = 1; want <= 32; ++want) {
+      if (want > 1 && (!may_split || steps / want < 6 || 2 * tiles * want > 9ull * cus)) break;
+      const uint32_t per = (steps + want - 1) / want, splits = (steps + per - 1) / per;
+      if (splits == tried) continue;
+      tried = splits;
+      if (s.bm == 64 && tiles * splits > (uint64_t)cus) break;
+      const double cost = strip_cost(s, rows, cols, splits, per, cus);
+      if (best_cost == 0 || cost < best_cost) {
+        best = StripPlan{i, splits, per};
+        best_cost = cost;
+      }
+    }
+  }
+  return best;
+}
+
+uint64_t strip_bytes(const StripPlan& p, uint32_t rows, uint32_t cols) {
+  return p.splits > 1 ? ((uint64_t)p.splits * rows * cols * 4 + 255) & ~uint64_t(255) : 0;
+}
+
+int strip_check(uint64_t reduction) {
+  if (reduction % 64) return mo::set_error(MO_E_INVALID, "strip kernels take reductions that are multiples of 64");
+  return 0;
+}
+
+// One strip call: C[rows][cols] from a reduction of A's columns.
+int strip_call(bool backward, uint64_t a, uint64_t w, uint64_t scale, uint64_t bias, uint64_t c, uint32_t rows,
+               uint32_t cols, uint32_t reduction, uint64_t workspace, uint64_t workspace_bytes, uint64_t stream) {
+  if (int rc = strip_check(reduction)) return rc;
+  if (workspace % 16) return mo::set_error(MO_E_INVALID, "workspace pointer must be 16-byte aligned");
+  GemmModule m;
+  if (int rc = gemm_module(&m)) return rc;
+  const StripPlan p = strip_plan(rows, cols, reduction / 64, m.cus, workspace != 0);
+  if (workspace && workspace_bytes < strip_bytes(p, rows, cols))
+    return mo::set_error(MO_E_INVALID, "workspace smaller than mo_int8_strip_workspace_bytes");
+  const Strip& s = kStrips[p.shape];
+  const uint64_t grid = div_up(rows, s.bm) * div_up(cols, s.bn) * p.splits;
+  if (grid >= (1ull << 31)) return mo::set_error(MO_E_INVALID, "grid too large");
+  const void* A = (const void*)a;
+  const void* W = (const void*)w;
+  const void* S = (const void*)scale;
   const void* Bi = (const void*)bias;
   void* C = (void*)c;
-  uint32_t rows = part.rows, n = cols, sp = part.splits;
-  void* rparams[] = {&Pc, &Bi, &C, &rows, &n, &sp};
-  const uint64_t lanes = (uint64_t)part.rows * (cols / 8);
-  e = hipModuleLaunchKernel(m.split_reduce, (uint32_t)((lanes + 255) / 256), 1, 1, 256, 1, 1, 0, (hipStream_t)stream,
-                            rparams, nullptr);
-  if (e != hipSuccess) return mo::set_hip_error((int)e, "int8 split reduction launch");
+  void* P = (void*)workspace;
+  int M = (int)rows, N = (int)cols, K = (int)reduction, splits = (int)p.splits, per = (int)p.split_steps;
+  void* params[] = {&A, &W, &S, &Bi, &C, &P, &M, &N, &K, &splits, &per};
+  const uint32_t threads = 64 * 4 * (s.bm == 128 ? s.k_groups : 1);  // 64-column tiles: one wave a K group
+  const hipError_t e = hipModuleLaunchKernel(m.strip[backward][p.shape], (uint32_t)grid, 1, 1, threads, 1, 1, 0,
+                                             (hipStream_t)stream, params, nullptr);
+  if (e != hipSuccess) return mo::set_hip_error((int)e, "int8 strip launch");
+  if (p.splits > 1) return launch_split_reduce(m, workspace, bias, c, rows, cols, p.splits, stream);
   return 0;
 }
 
@@ -373,6 +492,37 @@ int mo_int8_launch_plan(uint32_t rows, uint32_t cols, uint32_t reduction, uint32
     parts[5 * i + 4] = p[i].split_steps;
   }
   *n_parts = (uint32_t)n;
+  return 0;
+}
+
+uint64_t mo_int8_strip_workspace_bytes(uint32_t rows, uint32_t cols, uint32_t reduction) {
+  int cus = 0;
+  if (rows == 0 || cols == 0 || reduction == 0 || reduction % 64 || cu_count(&cus)) return 0;
+  return strip_bytes(strip_plan(rows, cols, reduction / 64, cus, true), rows, cols);
+}
+
+int mo_int8_strip_forward(uint64_t x, uint64_t w, uint64_t scale, uint64_t bias, uint64_t y, uint32_t rows,
+                          uint32_t in_features, uint32_t out_features, uint64_t workspace, uint64_t workspace_bytes,
+                          uint64_t stream) {
+  if (int rc = check(x, w, scale, y, rows, in_features, out_features)) return rc;
+  if (bias % 2) return mo::set_error(MO_E_INVALID, "bias pointer must be 2-byte aligned");
+  return strip_call(false, x, w, scale, bias, y, rows, out_features, in_features, workspace, workspace_bytes, stream);
+}
+
+int mo_int8_strip_backward(uint64_t dy, uint64_t w, uint64_t scale, uint64_t dx, uint32_t rows, uint32_t in_features,
+                           uint32_t out_features, uint64_t workspace, uint64_t workspace_bytes, uint64_t stream) {
+  if (int rc = check(dy, w, scale, dx, rows, in_features, out_features)) return rc;
+  return strip_call(true, dy, w, scale, 0, dx, rows, in_features, out_features, workspace, workspace_bytes, stream);
+}
+
+int mo_int8_strip_plan(uint32_t rows, uint32_t cols, uint32_t reduction, uint32_t cus, uint32_t may_split,
+                       uint32_t* plan) {
+  if (!plan) return mo::set_error(MO_E_INVALID, "null output pointer");
+  if (rows == 0 || cols == 0 || reduction == 0 || cus == 0) return mo::set_error(MO_E_INVALID, "empty shape");
+  if (int rc = strip_check(reduction)) return rc;
+  const StripPlan p = strip_plan(rows, cols, reduction / 64, (int)cus, may_split != 0);
+  const Strip& s = kStrips[p.shape];
+  plan[0] = s.bm, plan[1] = s.bn, plan[2] = s.k_groups, plan[3] = p.splits, plan[4] = p.split_steps;
   return 0;
 }
 

@@ -69,6 +69,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
 
 #define MO_LDS __attribute__((address_space(3)))
 
@@ -694,6 +695,410 @@ __device__ __forceinline__ void ws_body(const __bf16* __restrict__ A, const int8
   }
 }
 
+// ---- strips: calls with few rows ----
+// C[M][N] = A[M][K] . W'^T for calls that leave the 256 x 256 tile's grid short of the GPU or of
+// whole rounds, over weights as they are stored: forward W = weight [N][K], scales per column;
+// input gradient (kBwd) W = weight [K][N], scales per reduction index, no transposed copy.
+// K % 64 == 0; N % 16 == 0.
+//
+// What bounds such a call is not the matrix cores but how much of the GPU it reaches: 320 rows of
+// a 3072 x 3072 weight are 72 tiles of 128 x 128 on 256 CUs, each over a 48-step chain (30 us
+// where the products take 4; 15.7 here, four K groups on 64 x 64 tiles), 361 rows against a
+// 24576-long reduction 36 (274 us through the decoded weight and the library; 64 here, seven
+// splits of two K groups, 44 us of them at the MFMAs' rate). So the tile comes in five shapes (Strip) and the reduction is
+// shared out three ways, each where it costs least: over the K groups of a workgroup (WK, summed
+// through LDS at the end), over `splits` workgroups (fp32 planes, mo_int8_split_reduce), or not
+// at all. mo_gemm.cpp's cost model picks shape and splits.
+//
+// A workgroup is WN x WK waves over a (32 RT) x (32 CT WN) tile; wave (wn, wk) owns all rows and
+// 32 CT columns over K group wk's part of the reduction. Per step of 64, both operands go global
+// -> LDS by the buffer-load DMA path, A swizzled as in gemm_body, the weight as int8 bytes (half
+// the LDS and L2 traffic of a decoded tile); each wave decodes its own columns into the MFMA's B
+// fragments. Two LDS buffers an operand (64 KiB for the 128 x 256 tile), so two workgroups share a
+// CU and one computes while the other waits at its barrier.
+//   forward         16-byte chunks of a column's 64 bytes XOR-swizzled by column: a lane reads its
+//                   8 bytes of a slice, neighbouring slices in one 16-byte read.
+//   input gradient  64 rows of 32 CT WN bytes; ds_read_b64_tr_b8 (each group of 16 lanes
+//                   transposes 8 rows x 16 bytes) hands lane l the 8 reduction indices of column
+//                   l % 16, which is the B fragment; 32-byte units XOR-swizzled by row, so the 8
+//                   rows of a read fall on distinct banks. The step's 64 scales pass through a
+//                   register and are rounded to bf16 on their way into LDS, once a step.
+// Slice q of a step reads the A fragments of slice q + 1 and the weight bytes of slice q + 2, and
+// decodes slice q + 1 while its MFMAs run: five VALU behind each MFMA fill its shadow (all of a
+// slice's decode behind its last MFMAs cost 8 % more). After slice 2 the DMA of the next step
+// must have landed and the workgroup meets; slice 3 reads the next step's first slices and
+// refills the buffer just read. The products of an element are added in the order of the other
+// kernels (lane half h, chunk 4 h + q), so an unsplit, one-K-group call agrees with them bitwise.
+// With no decode the loop reaches 1 370-1 430 TFLOP/s, with no decode and no DMA 1 620, as it is
+// 1 200 (two workgroups a CU, 2 048 x 8 192 outputs): decode and DMA share the issue slots and the
+// power left by the MFMAs.
+template <int RT, int CT, int WN, int WK, bool kBwd, int kCap>
+__device__ __forceinline__ void strip_body(__bf16* a0, __bf16* a1, unsigned char* w0, unsigned char* w1, float* s0,
+                                           float* s1, const __bf16* __restrict__ A, const int8_t* __restrict__ W,
+                                           const float* __restrict__ scale, const __bf16* __restrict__ bias,
+                                           __bf16* __restrict__ C, float* __restrict__ P, int M, int N, int K, int m0,
+                                           int c0, int split, int splits, int split_steps) {
+  constexpr int kBM = 32 * RT, kBN = 32 * CT * WN;
+  // 1 KiB blocks of a K group's A tile (8 rows) and weight tile that each of its waves copies
+  constexpr int kAdma = kBM / 8 / WN, kWdma = kBN / 16 / WN, kDma = kAdma + kWdma;
+  static_assert(kBM % (8 * WN) == 0 && kBN % (16 * WN) == 0, "DMA blocks must divide over the waves");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave % WN, wk = wave / WN;
+  const int lr = lane & 31, h = lane >> 5;
+  // distinct objects per buffer, chosen at compile time: the compiler then knows which reads a
+  // DMA in flight can reach
+  auto abuf = [&](auto i) { return (MO_LDS __bf16*)(decltype(i)::value == 0 ? a0 : a1) + wk * kBM * kBR; };
+  auto wbuf = [&](auto i) { return (MO_LDS unsigned char*)(decltype(i)::value == 0 ? w0 : w1) + wk * kBN * kBR; };
+  auto sbuf = [&](auto i) { return (MO_LDS float*)(decltype(i)::value == 0 ? s0 : s1) + (kBwd ? wk * kBR : 0); };
+
+  // this K group's reduction [k0, k0 + klen); every group runs the same number of steps, those
+  // past its end on zeros
+  const int wg_k0 = split * split_steps * kBR, wg_len = min(split_steps * kBR, K - wg_k0);
+  const int steps = (wg_len / kBR + WK - 1) / WK;
+  const int k0 = wg_k0 + wk * steps * kBR, klen = max(0, min(steps * kBR, wg_len - wk * steps * kBR));
+  const bool any = klen > 0;
+  const rsrc_t ra_src = make_rsrc(A + (size_t)m0 * K + k0, any ? (uint32_t)((min(M - m0, kBM) * K - k0) * 2) : 0u);
+  const rsrc_t rw_src = kBwd ? make_rsrc(W + (size_t)k0 * N + c0, any ? (uint32_t)((klen - 1) * N + (N - c0)) : 0u)
+                             : make_rsrc(W + (size_t)c0 * K + k0, any ? (uint32_t)(min(N - c0, kBN) * K - k0) : 0u);
+  const rsrc_t rs_src = kBwd ? make_rsrc(scale + k0, any ? (uint32_t)klen * 4 : 0u) : make_rsrc(scale, (uint32_t)N * 4);
+
+  uint32_t a_off[kAdma], w_off[kWdma];
+#pragma unroll
+  for (int j = 0; j < kAdma; ++j) {
+    const int row = (wn * kAdma + j) * 8 + (lane >> 3);
+    a_off[j] = (uint32_t)(row * K + 8 * ((lane & 7) ^ ((row ^ (row >> 3)) & 7))) * 2;
+  }
+  // input gradient: XOR of a row's 32-byte units that spreads 8 rows over the 256 bytes of banks
+  auto unit = [](int row) { return kBN >= 256 ? row & 7 : kBN == 128 ? (row >> 1) & 3 : (row >> 2) & 1; };
+#pragma unroll
+  for (int j = 0; j < kWdma; ++j) {
+    const int block = wn * kWdma + j;
+    if (kBwd) {
+      const int at = block * 64 + lane, row = at / (kBN / 16), chunk = (at % (kBN / 16)) ^ (unit(row) << 1);
+      w_off[j] = c0 + 16 * chunk < N ? (uint32_t)(row * N + 16 * chunk) : kOob;
+    } else {
+      const int col = block * 16 + (lane >> 2);
+      w_off[j] = (uint32_t)(col * K + 16 * ((lane & 3) ^ ((col >> 2) & 3)));
+    }
+  }
+  int rd_a[2][4], rd_w[CT][4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) rd_a[p][q] = swz(32 * p + lr, 4 * h + q);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      if (kBwd) {
+        const int row = 32 * h + 8 * q + ((lane & 15) >> 1);
+        const int byte = 32 * (CT * wn + ct) + 16 * ((lane >> 4) & 1) + 8 * (lane & 1);
+        rd_w[ct][q] = row * kBN + (byte ^ (unit(row) << 5));
+      } else {
+        const int col = 32 * (CT * wn + ct) + lr;
+        rd_w[ct][q] = col * kBR + 16 * ((2 * h + (q >> 1)) ^ ((col >> 2) & 3)) + 8 * (q & 1);
+      }
+    }
+  }
+  float sf[CT];  // forward: bf16-rounded column scales
+  if (!kBwd) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const int n = c0 + 32 * (CT * wn + ct) + lr;
+      sf[ct] = bf16_round(__builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(rs_src, n < N ? n * 4 : (int)kOob, 0, 0)));
+    }
+  }
+
+  auto dma = [&](MO_LDS __bf16* As, MO_LDS unsigned char* Ws, int r0) {
+    const rsrc_t a = r0 < klen ? ra_src : make_rsrc(A, 0u), w = r0 < klen ? rw_src : make_rsrc(W, 0u);
+#pragma unroll
+    for (int j = 0; j < kAdma; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(a, (MO_LDS void*)(As + (wn * kAdma + j) * 512), 16, a_off[j], r0 * 2, 0,
+                                               0);
+#pragma unroll
+    for (int j = 0; j < kWdma; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w, (MO_LDS void*)(Ws + (wn * kWdma + j) * 1024), 16, w_off[j],
+                                               kBwd ? r0 * N : r0, 0, 0);
+  };
+  // input gradient: lane l's scale of the step at r0 (every wave of the group loads and stores the
+  // same 64)
+  auto load_scale = [&](int r0) {
+    const rsrc_t s = r0 < klen ? rs_src : make_rsrc(scale, 0u);
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s, lane * 4, r0 * 4, 0));
+  };
+
+  bf16x8 fa[2][RT], fb[2][CT];  // fragments of two slices
+  auto read_a = [&](const MO_LDS __bf16* As, int q, int slot) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) fa[slot][i] = *(const MO_LDS bf16x8*)(As + rd_a[i & 1][q] + (i >> 1) * 64 * kBR);
+  };
+  u32x2 wq[2][CT];  // weight bytes of two slices, and their scales (input gradient)
+  float sk[2][8];
+  auto read_w = [&](MO_LDS unsigned char* Ws, const MO_LDS float* Ss, int q, int slot) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      if (kBwd) {
+        const i32x2 v = __builtin_amdgcn_ds_read_tr8_b64_v2i32((MO_LDS i32x2*)(Ws + rd_w[ct][q]));
+        wq[slot][ct] = u32x2{(uint32_t)v[0], (uint32_t)v[1]};
+      } else {
+        wq[slot][ct] = *(const MO_LDS u32x2*)(Ws + rd_w[ct][q]);
+      }
+    }
+    if (kBwd) {
+      const float4 lo = *(const MO_LDS float4*)(Ss + 32 * h + 8 * q);
+      const float4 hi = *(const MO_LDS float4*)(Ss + 32 * h + 8 * q + 4);
+      float* k = sk[slot];
+      k[0] = lo.x, k[1] = lo.y, k[2] = lo.z, k[3] = lo.w, k[4] = hi.x, k[5] = hi.y, k[6] = hi.z, k[7] = hi.w;
+    }
+  };
+  auto decode_w = [&](int slot) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      bf16x8 f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = decode(wq[slot][ct][j >> 2], j & 3, kBwd ? sk[slot][j] : sf[ct]);
+      fb[slot][ct] = f;
+    }
+  };
+
+  f32x16 acc[RT][CT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) acc[i][ct] = f32x16{};
+
+  // The waves of the workgroup meet; a wave that shares its buffers with no other (WN == 1) needs
+  // only its own waits. No fence: the caller has waited for this wave's LDS accesses and DMA.
+  auto meet = [&] {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    if (WN > 1) {
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // Instruction interleave of slice q: an MFMA, then one LDS read, then the decode's VALU evenly
+  // (in slice 3, whose weight bytes were only just read, over the later MFMAs), the DMA in slice 3.
+  auto schedule = [&](auto qc) {
+    constexpr int q = decltype(qc)::value, kMf = RT * CT, kWreads = CT + (kBwd ? 2 : 0);
+    constexpr int kMfma = 0x008, kValu = 0x002, kDsRead = 0x100, kVmem = 0x020, kSalu = 0x004;
+    constexpr int kLead = q < 3 ? 0 : kMf * 3 / 8, kPer = (CT * 20 + kMf - kLead - 1) / (kMf - kLead);
+    if (q == 3) __builtin_amdgcn_sched_group_barrier(kDsRead, 2 * kWreads, 0);
+#pragma unroll
+    for (int m = 0; m < kMf; ++m) {
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      if (m < RT || (q < 2 && m < RT + kWreads)) __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+      if (q == 3) {
+        __builtin_amdgcn_sched_group_barrier(kSalu, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(kVmem, (kDma + (kBwd ? 1 : 0) + kMf - 1) / kMf, 0);
+      }
+      if (m >= kLead) __builtin_amdgcn_sched_group_barrier(kValu, kPer, 0);
+    }
+  };
+
+  // Step over buffer b at reduction r0; buffer b1 holds the next step.
+  float s_next = 0.f;
+  auto step = [&](auto b, auto b1, int r0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int cq = q & 1, nq = cq ^ 1;
+      if (q < 3) read_a(abuf(b), q + 1, nq);
+      if (q < 2) read_w(wbuf(b), sbuf(b), q + 2, cq);
+      if (q == 3) {
+        read_w(wbuf(b1), sbuf(b1), 0, 0);
+        read_a(abuf(b1), 0, nq);
+        read_w(wbuf(b1), sbuf(b1), 1, 1);
+        if (kBwd) {  // step r0 + 128's scales, loaded a step ago; then the next load
+          sbuf(b)[lane] = bf16_round(s_next);
+          s_next = load_scale(r0 + 3 * kBR);
+        }
+        dma(abuf(b), wbuf(b), r0 + 2 * kBR);
+      }
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+          acc[i][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[cq][i], fb[cq][ct], acc[i][ct], 0, 0, 0);
+      decode_w(nq);
+      if (q == 0) schedule(std::integral_constant<int, 0>{});
+      if (q == 1) schedule(std::integral_constant<int, 1>{});
+      if (q == 2) schedule(std::integral_constant<int, 2>{});
+      if (q == 3) schedule(std::integral_constant<int, 3>{});
+      __builtin_amdgcn_sched_barrier(0);
+      if (q == 2) {
+        // every load of this wave has landed (the next step's among them) and its reads of buffer
+        // b are done; then all waves'
+        __builtin_amdgcn_s_waitcnt(wait_vm(0, 0));
+        meet();
+      }
+    }
+  };
+
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  dma(abuf(B0{}), wbuf(B0{}), 0);
+  if (kBwd) {
+    const float first = load_scale(0), second = load_scale(kBR);
+    s_next = load_scale(2 * kBR);
+    sbuf(B0{})[lane] = bf16_round(first);
+    sbuf(B1{})[lane] = bf16_round(second);
+  }
+  dma(abuf(B1{}), wbuf(B1{}), kBR);
+  __builtin_amdgcn_s_waitcnt(wait_vm(kDma, 0));
+  meet();
+  read_w(wbuf(B0{}), sbuf(B0{}), 0, 0);
+  read_a(abuf(B0{}), 0, 0);
+  read_w(wbuf(B0{}), sbuf(B0{}), 1, 1);
+  decode_w(0);
+  for (int s = 0; s < steps; s += 2) {  // an odd count runs one more step, on zeros
+    step(B0{}, B1{}, s * kBR);
+    step(B1{}, B0{}, (s + 1) * kBR);
+  }
+
+  if constexpr (WK > 1) {
+    // K groups 1, 2, .. into group 0, in that order, through the A buffers: kFit row tiles of a
+    // group's waves fit one of them
+    constexpr int kFit = kCap * 2 / (CT * 4096 * WN);
+    static_assert(kFit >= 1, "a row tile of every wave must fit an A buffer");
+    auto at = [&](int i, int i0, int ct) {
+      return (MO_LDS float*)(i - i0 >= kFit ? a1 : a0) + ((wn * kFit + (i - i0) % kFit) * CT + ct) * 1024 + lane * 4;
+    };
+    __builtin_amdgcn_s_waitcnt(wait_vm(0, 0));
+    __syncthreads();
+#pragma unroll
+    for (int g = 1; g < WK; ++g) {
+#pragma unroll
+      for (int i0 = 0; i0 < RT; i0 += 2 * kFit) {
+        const int i1 = i0 + 2 * kFit < RT ? i0 + 2 * kFit : RT;
+        if (wk == g) {
+#pragma unroll
+          for (int i = i0; i < i1; ++i)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                *(MO_LDS float4*)(at(i, i0, ct) + r * 256) =
+                    make_float4(acc[i][ct][4 * r], acc[i][ct][4 * r + 1], acc[i][ct][4 * r + 2], acc[i][ct][4 * r + 3]);
+        }
+        __syncthreads();
+        if (wk == 0) {
+#pragma unroll
+          for (int i = i0; i < i1; ++i)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const float4 v = *(const MO_LDS float4*)(at(i, i0, ct) + r * 256);
+                acc[i][ct][4 * r] += v.x;
+                acc[i][ct][4 * r + 1] += v.y;
+                acc[i][ct][4 * r + 2] += v.z;
+                acc[i][ct][4 * r + 3] += v.w;
+              }
+        }
+        __syncthreads();
+      }
+    }
+    if (wk != 0) return;
+  }
+
+  const int cw = c0 + 32 * CT * wn;  // the wave's first column
+  if (splits > 1) {
+    const rsrc_t rp_src = make_rsrc(P + ((size_t)split * M + m0) * N, (uint32_t)(min(M - m0, kBM) * N * 4));
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const int col = cw + 32 * ct + lr;
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+          const float v = acc[i][ct][r];  // through a scalar, as in ws_body
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), rp_src,
+                                                col < N ? (int)((uint32_t)(row * N + col) * 4) : (int)kOob, 0, 0);
+        }
+    }
+    return;
+  }
+  const rsrc_t rc_src = make_rsrc(C + (size_t)m0 * N, (uint32_t)(min(M - m0, kBM) * N * 2));
+  const rsrc_t rbias_src = make_rsrc(bias, bias ? (uint32_t)N * 2 : 0u);
+  float b[CT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    const int col = cw + 32 * ct + lr;
+    b[ct] = (float)__builtin_bit_cast(
+        __bf16, (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rbias_src, col < N ? col * 2 : (int)kOob, 0, 0));
+  }
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row0 = i * 32 + 8 * (r >> 2) + (r & 3);
+      const unsigned int x = __builtin_bit_cast(unsigned short, (__bf16)(acc[i][0][r] + b[0]));
+      if constexpr (CT == 1) {
+        const int col = cw + lr;
+        __builtin_amdgcn_raw_buffer_store_b16(
+            (unsigned short)x, rc_src, col < N ? (int)((uint32_t)((row0 + 4 * h) * N + col) * 2) : (int)kOob, 0, 0);
+      } else {  // the lane-half swap of ws_body: 128-byte row pieces
+        const int col = cw + lane;
+        const unsigned int y = __builtin_bit_cast(unsigned short, (__bf16)(acc[i][1][r] + b[1]));
+        const auto sw = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        __builtin_amdgcn_raw_buffer_store_b16((unsigned short)sw[0], rc_src,
+                                              col < N ? (int)((uint32_t)(row0 * N + col) * 2) : (int)kOob, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b16((unsigned short)sw[1], rc_src,
+                                              col < N ? (int)((uint32_t)((row0 + 4) * N + col) * 2) : (int)kOob, 0, 0);
+      }
+    }
+}
+
+// The strip kernels. Workgroups of full row tiles come first, then those of the last, shorter row
+// tile, which run a body of fewer row tiles: they cost less and fill the last round (1 327 rows of
+// a 24 576-wide output, 10 full row tiles and 47 rows: 205 -> 196 us). Each part is numbered XCD-
+// aware, by split, then in groups of kGroupM row tiles.
+template <int RT, int CT, int WN, int WK, bool kBwd>
+__device__ __forceinline__ void strip_main(const __bf16* __restrict__ A, const int8_t* __restrict__ W,
+                                           const float* __restrict__ scale, const __bf16* __restrict__ bias,
+                                           __bf16* __restrict__ C, float* __restrict__ P, int M, int N, int K,
+                                           int splits, int split_steps) {
+  static_assert(CT <= 2 && RT <= 4, "epilogue and tail bodies");
+  constexpr int kBM = 32 * RT, kBN = 32 * CT * WN, kCap = WK * kBM * kBR;
+  __shared__ __attribute__((aligned(16))) __bf16 a0[kCap];
+  __shared__ __attribute__((aligned(16))) __bf16 a1[kCap];
+  __shared__ __attribute__((aligned(16))) unsigned char w0[WK * kBN * kBR];
+  __shared__ __attribute__((aligned(16))) unsigned char w1[WK * kBN * kBR];
+  __shared__ __attribute__((aligned(16))) float s0[kBwd ? WK * kBR : 4];
+  __shared__ __attribute__((aligned(16))) float s1[kBwd ? WK * kBR : 4];
+  const int tiles_c = (N + kBN - 1) / kBN, full_m = M / kBM;
+  const int full = full_m * tiles_c * splits;  // workgroups of full row tiles
+  const bool last = (int)blockIdx.x >= full;
+  const int items = last ? (int)gridDim.x - full : full;
+  int t;
+  {
+    const int b = blockIdx.x - (last ? full : 0), xcd = b % kXcds, idx = b / kXcds;
+    const int per = items / kXcds, rem = items % kXcds;
+    t = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+  }
+  const int tiles = items / splits, rows_m = last ? 1 : full_m;
+  const int split = t / tiles;
+  t -= split * tiles;
+  const int first_m = (t / (kGroupM * tiles_c)) * kGroupM, gm = min(rows_m - first_m, kGroupM);
+  const int in_group = t % (kGroupM * tiles_c);
+  const int m0 = (last ? full_m : first_m + in_group % gm) * kBM, c0 = (in_group / gm) * kBN;
+  auto body = [&](auto rt) {
+    strip_body<decltype(rt)::value, CT, WN, WK, kBwd, kCap>(a0, a1, w0, w1, s0, s1, A, W, scale, bias, C, P, M, N, K, m0,
+                                                            c0, split, splits, split_steps);
+  };
+  const int rt = last ? (M - m0 + 31) / 32 : RT;
+  if constexpr (RT > 3)
+    if (rt == 3) return body(std::integral_constant<int, 3>{});
+  if constexpr (RT > 2)
+    if (rt == 2) return body(std::integral_constant<int, 2>{});
+  if constexpr (RT > 1)
+    if (rt == 1) return body(std::integral_constant<int, 1>{});
+  body(std::integral_constant<int, RT>{});
+}
+
 // Configurations: forward 256 x 256 over 2 x 4 waves (two waves a SIMD); input gradient
 // 256 x 256 over 2 x 2 waves; both directions 128 x 128 over 2 x 2 waves for grids too small
 // or too ragged for the large tile.
@@ -739,6 +1144,24 @@ extern "C" __global__ __launch_bounds__(256) void mo_int8_ws_kscale_split(const 
                                                                             int split_steps) {
   mo_gemm::ws_body<true, true>(A, Bq, scale, nullptr, nullptr, P, M, N, K, tiles_m, splits, split_steps);
 }
+
+// Strips (kStrips in mo_gemm.cpp): row tile x column tile, K groups. Two waves a SIMD at least.
+#define MO_STRIP(NAME, RT, CT, WN, WK)                                                                              \
+  extern "C" __global__ __launch_bounds__(64 * WN * WK, 2) void mo_int8_strip_fwd_##NAME(                           \
+      const __bf16* A, const int8_t* W, const float* scale, const __bf16* bias, __bf16* C, float* P, int M, int N,  \
+      int K, int splits, int split_steps) {                                                                         \
+    mo_gemm::strip_main<RT, CT, WN, WK, false>(A, W, scale, bias, C, P, M, N, K, splits, split_steps);              \
+  }                                                                                                                 \
+  extern "C" __global__ __launch_bounds__(64 * WN * WK, 2) void mo_int8_strip_bwd_##NAME(                           \
+      const __bf16* A, const int8_t* W, const float* scale, const __bf16* bias, __bf16* C, float* P, int M, int N,  \
+      int K, int splits, int split_steps) {                                                                         \
+    mo_gemm::strip_main<RT, CT, WN, WK, true>(A, W, scale, bias, C, P, M, N, K, splits, split_steps);               \
+  }
+MO_STRIP(128x256, 4, 2, 4, 1)
+MO_STRIP(128x256k2, 4, 2, 4, 2)
+MO_STRIP(128x128, 4, 1, 4, 1)
+MO_STRIP(64x64k4, 2, 2, 1, 4)
+MO_STRIP(32x64k4, 1, 2, 1, 4)
 
 // C[rows][cols] = bf16(P[0] + P[1] + ... + P[splits - 1] (+ bias)), the planes of a split
 // reduction added in split order, so the result does not depend on which workgroup finished

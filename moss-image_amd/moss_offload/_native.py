@@ -15,7 +15,7 @@ import torch  # noqa: F401  (must be imported before the library, see module doc
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libmoss_offload.so"
 
-MO_ABI_VERSION = 21
+MO_ABI_VERSION = 22
 MO_MAX_DIMS = 8
 
 MO_E_INVALID = 1001
@@ -259,6 +259,13 @@ SIGNATURES: dict[str, tuple] = {
     "mo_int8_linear_backward": (ctypes.c_int, [_u64, _u64, _u64, _u64, ctypes.c_uint32, ctypes.c_uint32,
                                                ctypes.c_uint32, _u64, _u64, _u64]),
     "mo_int8_backward_workspace_bytes": (_u64, [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32]),
+    "mo_int8_strip_forward": (ctypes.c_int, [_u64, _u64, _u64, _u64, _u64, ctypes.c_uint32, ctypes.c_uint32,
+                                             ctypes.c_uint32, _u64, _u64, _u64]),
+    "mo_int8_strip_backward": (ctypes.c_int, [_u64, _u64, _u64, _u64, ctypes.c_uint32, ctypes.c_uint32,
+                                              ctypes.c_uint32, _u64, _u64, _u64]),
+    "mo_int8_strip_workspace_bytes": (_u64, [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32]),
+    "mo_int8_strip_plan": (ctypes.c_int, [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32,
+                                          ctypes.c_uint32, _P(ctypes.c_uint32)]),
     "mo_int8_set_kernel": (ctypes.c_int, [ctypes.c_uint32]),
     "mo_int8_launch_plan": (ctypes.c_int, [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32,
                                            ctypes.c_uint32, _P(ctypes.c_uint32), _P(ctypes.c_uint32)]),

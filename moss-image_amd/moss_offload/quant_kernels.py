@@ -2,11 +2,14 @@
 ``training/quant_kernels.py`` (:100-228, ``triton_int8_linear_forward/backward``).
 
 The GEMMs are hand-written gfx950 kernels in ``csrc/mo_gemm.hip`` (bf16 MFMA; the int8
-weight decoded to bf16 in registers on its way into the MFMA), reached through
-``mo_int8_linear_forward`` and ``mo_int8_linear_backward``. From ``LIBRARY_ROWS`` rows or
-``LIBRARY_WEIGHT`` weight elements up, a call whose reduction is not long against its output
-width instead decodes the weight in one HIP pass (``mo_int8_decode``) and runs the same library
-GEMM as the eager path, bit for bit equal to it and faster by the decode. Backend selection mirrors the reference's ``auto | eager | triton``
+weight decoded to bf16 in registers on its way into the MFMA): the strip kernels for calls with
+few rows (``mo_int8_strip_forward`` / ``backward``), large tiles above them
+(``mo_int8_linear_forward`` / ``backward``). From ``LIBRARY_ROWS`` rows or ``LIBRARY_WEIGHT``
+weight elements up, a call above the strips whose reduction is not long against its output width
+instead decodes the weight in one HIP pass (``mo_int8_decode``) and runs the same library GEMM as
+the eager path, bit for bit equal to it and faster by the decode.
+
+Backend selection mirrors the reference's ``auto | eager | triton``
 with ``hip`` in place of ``triton``: ``auto`` takes the HIP kernels whenever the call is
 supported (bf16 activations and weight dtype on a HIP device, int8 weights, fp32 scales,
 feature sizes multiples of 16, contiguous operands) and the eager path otherwise; an explicit
@@ -80,25 +83,49 @@ def decode(weight: torch.Tensor, scale: torch.Tensor, dtype: torch.dtype) -> tor
     return weight.to(dtype) * scale.to(dtype)[:, None]
 
 
-# A call with at least LIBRARY_ROWS rows, or a weight of at least LIBRARY_WEIGHT elements,
-# decodes the weight once (mo_int8_decode) and runs the library GEMM on it, unless its
-# reduction is at least LONG_REDUCTION times its output width and the fused kernels' launch
-# plan splits that reduction (rows that do not fill a round of large tiles): there the fused
-# kernels run. Any other call runs the fused kernels. Measured on MI355X, library time / fused
-# time (forward, input gradient):
-#   rows:                 256        512        1024       2048       4096       8192       17792
-#   qkvo 3072x3072       1.19 0.84  0.97 1.07  0.98 1.10  0.90 0.93  0.89 0.75  0.91 0.89  0.86 0.90
-#   up_gate 24576x3072   1.46 2.04  1.20 2.01  1.08 1.56  0.98 1.28  0.88 0.70  0.85 0.86  0.83 1.04
-#   down 3072x12288      1.54 0.97  1.50 0.90  1.20 0.87  1.09 0.91  0.74 0.88  0.90 0.89  1.04 0.91
-# The rule takes the fused kernels for up_gate's input gradient (24576-long reduction) and
-# down's forward (12288) at 256-2048 and 17792 rows, where the library's GEMM runs its weakest
-# and the split reduction fills the GPU; the library otherwise. On square and wide shapes the
-# library's MFMA loop runs 10-15 % faster than the fused kernels' (which also decode each
-# weight tile again for every row tile).
+# Calls with few rows run the strip kernels (mo_int8_strip_*, reductions of whole steps of 64). The
+# other paths pay for a decode of the whole weight (8 to 40 us), or for a grid of large tiles that
+# does not fill the GPU. Measured on MI355X, us, strip / fused / library:
+#   rows                       320           700           1000          1450          2100          2693          4608
+#   forward
+#    3072 from 3072         15/28/31      25/31/32      30/35/36      41/48/46      43/54/49      54/78/55     82/102/71
+#    3072 from 12288       36/109/61      62/68/92     81/85/100   117/112/134   149/150/275   205/295/307   308/413/258
+#    16384 from 3072        37/46/58      73/81/84      92/85/98   134/144/145   201/197/230   252/233/329   396/389/442
+#    24576 from 3072        56/76/85   108/117/147   136/139/161   209/213/219   288/282/298   367/370/396   599/589/608
+#   input gradient
+#    3072 from 3072         15/38/31      26/37/37      31/42/50      43/56/49      42/62/53      60/94/73     82/115/81
+#    3072 from 24576      58/284/205   108/148/267   148/174/275   220/257/344   287/349/421   404/701/651   611/931/833
+#    12288 from 3072        35/53/54      64/93/72      77/96/90   119/141/153   155/173/160   196/224/197   302/339/313
+# - input gradients below STRIP_ROWS_BACKWARD rows, and below STRIP_LONG_ROWS where the reduction is
+#   at least LONG_REDUCTION times the output width, for which the library's kernel is weak (8192
+#   rows of 3072 from 24576: strip 1038, library 931 on the transposed weight);
+# - forwards below STRIP_ROWS rows, and up to STRIP_ROWS_NARROW while their 128 x 256 tiles fill half
+#   a round of the CUs but hardly more than one (past it a second round starts: 3300 rows of 3072 from 8192 take
+#   175, the library 143; under half a round the large tiles split the reduction as well and the
+#   two are within 10 %: 2047 rows of 1040 from 3072, 28 / 31 / 31). Long reductions that the fused
+#   plan splits stay there from STRIP_LONG_ROWS_FORWARD rows (1700 rows of 3072 from 12288: 129 / 126).
+STRIP_ROWS = 1536
+STRIP_LONG_ROWS_FORWARD = 1280
+STRIP_TILES, STRIP_ROWS_NARROW = (128, 264), 2816
+STRIP_ROWS_BACKWARD = 2560
+STRIP_LONG_ROWS = 6144
+# Any other call with at least LIBRARY_ROWS rows, or a weight of at least LIBRARY_WEIGHT elements,
+# decodes the weight once (mo_int8_decode) and runs the library GEMM on it, unless its reduction is
+# at least LONG_REDUCTION times its output width and the fused kernels' launch plan splits that
+# reduction (rows that do not fill a round of large tiles): there the fused kernels run, as for any
+# call left. Measured, library time / fused time (forward, input gradient):
+#   rows:                4096       8192       17792
+#   qkvo 3072x3072       0.89 0.75  0.91 0.89  0.86 0.90
+#   up_gate 24576x3072   0.88 0.70  0.85 0.86  0.83 1.04
+#   down 3072x12288      0.74 0.88  0.90 0.89  1.04 0.91
+# The rule takes the fused kernels for up_gate's input gradient (24576-long reduction) and down's
+# forward (12288) at 17792 rows, where the library's GEMM runs its weakest and the split reduction
+# fills the GPU. On square and wide shapes the library's MFMA loop runs 10-15 % faster than the
+# fused kernels' (which also decode each weight tile again for every row tile).
 LIBRARY_ROWS = 2048
 LIBRARY_WEIGHT = 16 << 20
 LONG_REDUCTION = 4
-PATHS = ("auto", "fused", "library")
+PATHS = ("auto", "fused", "library", "strip")
 
 
 def decode_hip(weight: torch.Tensor, scale: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -112,17 +139,39 @@ def decode_hip(weight: torch.Tensor, scale: torch.Tensor, *, out: torch.Tensor |
     return out
 
 
-def _library(rows: int, weight: torch.Tensor, path: str, reduction: int, width: int, split) -> bool:
-    """Whether a call takes the library path; ``split()`` tells whether the fused plan splits a
-    reduction (asked only when the rule needs it)."""
+def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: int, backward: bool) -> str:
+    """The path a call takes: ``strip``, ``library`` or ``fused``."""
 
     if path not in PATHS:
         raise ValueError(f"path must be one of {PATHS}")
     if path != "auto":
-        return path == "library"
+        return path
+    long_reduction = reduction >= LONG_REDUCTION * width
+    if reduction % 64 == 0 and _strips(rows, reduction, width, backward, long_reduction):
+        return "strip"
     if rows < LIBRARY_ROWS and weight.numel() < LIBRARY_WEIGHT:
+        return "fused"
+    return "fused" if long_reduction and _splits(rows, width, reduction, backward) else "library"
+
+
+def _strips(rows: int, reduction: int, width: int, backward: bool, long_reduction: bool) -> bool:
+    """Whether a call runs the strip kernels (see ``STRIP_ROWS``)."""
+
+    if backward:
+        return rows < (STRIP_LONG_ROWS if long_reduction else STRIP_ROWS_BACKWARD)
+    if long_reduction and rows >= STRIP_LONG_ROWS_FORWARD and _splits(rows, width, reduction, False):
         return False
-    return not (reduction >= LONG_REDUCTION * width and split())
+    tiles = -(-rows // 128) * -(-width // 256)
+    return rows < STRIP_ROWS or (rows <= STRIP_ROWS_NARROW and STRIP_TILES[0] <= tiles <= STRIP_TILES[1])
+
+
+def _splits(rows: int, width: int, reduction: int, backward: bool) -> bool:
+    """Whether the fused kernels' launch plan splits the call's reduction."""
+
+    lib = _native.load()
+    if not backward:
+        return lib.mo_int8_forward_workspace_bytes(rows, reduction, width) > 0
+    return lib.mo_int8_backward_workspace_bytes(rows, width, reduction) > (width * reduction + 255) // 256 * 256
 
 
 def _stream(tensor: torch.Tensor) -> int:
@@ -138,13 +187,20 @@ def _output(out: torch.Tensor | None, shape: tuple[int, int], device: torch.devi
     return out.view(shape)
 
 
+def _workspace(nbytes: int, device: torch.device) -> torch.Tensor | None:
+    # fp32 partial sums of split reductions, the transposed weight of the fused input gradient: freed
+    # to the caching allocator after the call; stream order keeps it alive for the kernels
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+
+
 def int8_linear_forward(tokens: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor,
                         bias: torch.Tensor | None = None, *, out: torch.Tensor | None = None,
                         path: str = "auto") -> torch.Tensor:
-    """``tokens @ decode(weight).T (+ bias)``; the call must be supported. ``path``: ``fused`` (the
-    MFMA kernels), ``library`` (``decode_hip``, then the same ``addmm``/``mm`` as the reference's
-    eager path, bit for bit), ``auto`` (library from ``LIBRARY_ROWS`` rows or ``LIBRARY_WEIGHT``
-    weight elements up)."""
+    """``tokens @ decode(weight).T (+ bias)``; the call must be supported. ``path``: ``strip`` (the
+    MFMA kernels for few rows; ``in_features`` a multiple of 64), ``fused`` (the MFMA kernels on
+    large tiles), ``library`` (``decode_hip``, then the same ``addmm``/``mm`` as the reference's
+    eager path, bit for bit), ``auto`` (by rows and shape, see ``STRIP_ROWS`` and
+    ``LIBRARY_ROWS``)."""
 
     lib = _native.load()
     matrix = tokens.reshape(-1, tokens.shape[-1]).contiguous()
@@ -152,8 +208,8 @@ def int8_linear_forward(tokens: torch.Tensor, weight: torch.Tensor, scale: torch
     out_features = weight.shape[0]
     if bias is not None:
         bias = bias.to(torch.bfloat16).contiguous()
-    nbytes = lib.mo_int8_forward_workspace_bytes(rows, in_features, out_features)
-    if _library(rows, weight, path, in_features, out_features, lambda: nbytes > 0):
+    route = _route(path, rows, weight, in_features, out_features, False)
+    if route == "library":
         decoded = decode_hip(weight, scale)
         if out is None:
             # the eager path's own call (F.linear): with an output buffer, PyTorch-ROCm picks
@@ -165,16 +221,16 @@ def int8_linear_forward(tokens: torch.Tensor, weight: torch.Tensor, scale: torch
                 torch.addmm(bias, matrix, decoded.t(), out=out)
         return result.reshape(*tokens.shape[:-1], out_features)
     out = _output(out, (rows, out_features), tokens.device, "output")
-    # fp32 partial sums of split reductions (freed to the caching allocator after the call;
-    # stream order keeps them alive for the kernels)
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=tokens.device) if nbytes else None
-    _native.check(
-        "mo_int8_linear_forward",
-        lib.mo_int8_linear_forward(matrix.data_ptr(), weight.data_ptr(), scale.data_ptr(),
-                                   0 if bias is None else bias.data_ptr(), out.data_ptr(), rows, in_features,
-                                   out_features, 0 if workspace is None else workspace.data_ptr(), nbytes,
-                                   _stream(tokens)),
-    )
+    if route == "strip":
+        name, call = "mo_int8_strip_forward", lib.mo_int8_strip_forward
+        nbytes = lib.mo_int8_strip_workspace_bytes(rows, out_features, in_features)
+    else:
+        name, call = "mo_int8_linear_forward", lib.mo_int8_linear_forward
+        nbytes = lib.mo_int8_forward_workspace_bytes(rows, in_features, out_features)
+    workspace = _workspace(nbytes, tokens.device)
+    _native.check(name, call(matrix.data_ptr(), weight.data_ptr(), scale.data_ptr(),
+                             0 if bias is None else bias.data_ptr(), out.data_ptr(), rows, in_features, out_features,
+                             0 if workspace is None else workspace.data_ptr(), nbytes, _stream(tokens)))
     return out.reshape(*tokens.shape[:-1], out_features)
 
 
@@ -182,29 +238,30 @@ def int8_linear_backward(gradient: torch.Tensor, weight: torch.Tensor, scale: to
                          input_shape: torch.Size, *, out: torch.Tensor | None = None,
                          path: str = "auto") -> torch.Tensor:
     """``gradient @ decode(weight)``: the input gradient of the frozen int8 linear (``path`` as in
-    ``int8_linear_forward``)."""
+    ``int8_linear_forward``; ``strip`` needs ``out_features`` a multiple of 64)."""
 
     lib = _native.load()
     matrix = gradient.reshape(-1, gradient.shape[-1]).to(torch.bfloat16).contiguous()
     rows, out_features = matrix.shape
     in_features = weight.shape[1]
-    nbytes = lib.mo_int8_backward_workspace_bytes(rows, in_features, out_features)
-    transposed = (in_features * out_features + 255) // 256 * 256
-    if _library(rows, weight, path, out_features, in_features, lambda: nbytes > transposed):
+    route = _route(path, rows, weight, out_features, in_features, True)
+    if route == "library":
         if out is None:  # the eager path's call (see int8_linear_forward)
             return matrix.matmul(decode_hip(weight, scale)).reshape(input_shape)
         out = _output(out, (rows, in_features), gradient.device, "input-gradient")
         torch.mm(matrix, decode_hip(weight, scale), out=out)
         return out.reshape(input_shape)
     out = _output(out, (rows, in_features), gradient.device, "input-gradient")
-    # the transposed int8 weight for the large tiles and the partial sums of split reductions
-    # (freed to the caching allocator after the call; stream order keeps it alive for the kernels)
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=gradient.device)
-    _native.check(
-        "mo_int8_linear_backward",
-        lib.mo_int8_linear_backward(matrix.data_ptr(), weight.data_ptr(), scale.data_ptr(), out.data_ptr(), rows,
-                                    in_features, out_features, workspace.data_ptr(), nbytes, _stream(gradient)),
-    )
+    if route == "strip":
+        name, call = "mo_int8_strip_backward", lib.mo_int8_strip_backward
+        nbytes = lib.mo_int8_strip_workspace_bytes(rows, in_features, out_features)
+    else:
+        name, call = "mo_int8_linear_backward", lib.mo_int8_linear_backward
+        nbytes = lib.mo_int8_backward_workspace_bytes(rows, in_features, out_features)
+    workspace = _workspace(nbytes, gradient.device)
+    _native.check(name, call(matrix.data_ptr(), weight.data_ptr(), scale.data_ptr(), out.data_ptr(), rows, in_features,
+                             out_features, 0 if workspace is None else workspace.data_ptr(), nbytes,
+                             _stream(gradient)))
     return out.reshape(input_shape)
 
 
@@ -224,6 +281,18 @@ def launch_plan(rows: int, cols: int, reduction: int, cus: int, kernel: str = "r
     names = ("large", "small", "split")
     return [{"tile": names[raw[5 * i]], "row0": raw[5 * i + 1], "rows": raw[5 * i + 2], "splits": raw[5 * i + 3],
              "split_steps": raw[5 * i + 4]} for i in range(n.value)]
+
+
+def strip_plan(rows: int, cols: int, reduction: int, cus: int, may_split: bool = True) -> dict:
+    """The strip kernels' plan (``mo_int8_strip_plan``): ``{"rows", "cols"}`` of the output tile,
+    ``"k_groups"`` of a workgroup, ``"splits"`` and ``"split_steps"`` of the reduction."""
+
+    import ctypes
+
+    raw = (ctypes.c_uint32 * 5)()
+    _native.check("mo_int8_strip_plan", _native.load().mo_int8_strip_plan(rows, cols, reduction, cus, int(may_split),
+                                                                          raw))
+    return dict(zip(("rows", "cols", "k_groups", "splits", "split_steps"), raw))
 
 
 def set_kernel(kernel: str) -> None:

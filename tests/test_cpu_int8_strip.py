@@ -1,0 +1,53 @@
+"""The strip kernels' plan (``mo_int8_strip_plan``, host only): the shapes the GPU test's cases
+take, and what every plan must keep."""
+
+from __future__ import annotations
+
+import random
+
+import pytest
+
+from moss_offload import _native, quant_kernels as qk
+
+CUS = 256  # MI355X
+
+# rows, output columns, reduction; tile rows, tile columns, K groups, splits, steps per split
+CASES = [
+    (1, 16, 64, 32, 64, 4, 1, 1),
+    (33, 1040, 3072, 32, 64, 4, 6, 8),
+    (180, 2064, 4160, 32, 64, 4, 1, 65),
+    (97, 4112, 576, 64, 64, 4, 1, 9),
+    (390, 2064, 704, 64, 64, 4, 1, 11),
+    (1087, 8208, 512, 128, 128, 1, 1, 8),
+    (481, 2064, 2112, 128, 128, 1, 3, 11),
+    (700, 6160, 1024, 128, 256, 1, 1, 16),
+    (1985, 2832, 1088, 128, 256, 1, 1, 17),
+    (300, 4112, 9216, 128, 256, 1, 5, 29),
+    (700, 3072, 12288, 128, 256, 2, 3, 64),
+    (159, 24576, 3072, 128, 256, 2, 1, 48),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_cases_take_their_shapes(case) -> None:
+    assert tuple(qk.strip_plan(*case[:3], CUS).values()) == case[3:]
+
+
+def test_every_plan_keeps_its_invariants() -> None:
+    rng = random.Random(11)
+    tiles = {(128, 256, 1), (128, 256, 2), (128, 128, 1), (64, 64, 4), (32, 64, 4)}
+    for _ in range(3000):
+        rows = rng.choice([rng.randrange(1, 600), rng.randrange(1, 40000)])
+        cols = 16 * rng.randrange(1, 2048)
+        steps = rng.randrange(1, 500)
+        cus = rng.choice([256, 304, 80])
+        p = qk.strip_plan(rows, cols, 64 * steps, cus)
+        assert (p["rows"], p["cols"], p["k_groups"]) in tiles
+        assert (p["splits"] - 1) * p["split_steps"] < steps <= p["splits"] * p["split_steps"]
+        grid = -(-rows // p["rows"]) * -(-cols // p["cols"]) * p["splits"]
+        assert p["splits"] == 1 or (p["splits"] <= 32 and p["split_steps"] >= 6 and 2 * grid <= 9 * cus)
+        assert p["rows"] != 64 or grid <= cus
+        alone = qk.strip_plan(rows, cols, 64 * steps, cus, may_split=False)
+        assert alone["splits"] == 1 and alone["split_steps"] == steps
+    with pytest.raises(_native.EngineError):
+        qk.strip_plan(64, 64, 80, CUS)

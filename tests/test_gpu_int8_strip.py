@@ -1,0 +1,89 @@
+"""The strip kernels (mo_int8_strip_forward / backward): every tile shape, tails, splits.
+
+Each case is held to the fp64 product of the decoded weight within the bound of fp32 accumulation
+plus the final bf16 rounding, in both directions. The sizes put a ragged edge everywhere one can
+be: last row tiles of one to four 32-row tiles, output columns that end inside a column tile, K
+groups of unequal or no steps, odd step counts, a last split shorter than the others.
+``tests/test_cpu_int8_strip.py`` pins which shape the plan gives each case.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from moss_offload import _native, quant_kernels
+
+from gpu_util import requires_gpu
+from test_cpu_int8_strip import CASES
+from test_gpu_int8_gemm import DEV, _operands, _within_accumulation_bound
+
+pytestmark = requires_gpu
+
+
+@pytest.mark.parametrize("rows,cols,reduction", [c[:3] for c in CASES])
+@pytest.mark.parametrize("direction", ["forward", "bias", "backward"])
+def test_strip_matches_fp64_reference(rows, cols, reduction, direction) -> None:
+    if direction == "backward":
+        x, w, scale, b = _operands(rows, reduction, cols, seed=rows + cols)
+        w, scale = _operands(1, cols, reduction, seed=rows + 3 * cols)[1:3]  # [out = reduction][in = cols]
+        got = quant_kernels.int8_linear_backward(x, w, scale, torch.Size((rows, cols)), path="strip")
+        again = quant_kernels.int8_linear_backward(x, w, scale, torch.Size((rows, cols)), path="strip")
+        decoded = quant_kernels.decode(w, scale, torch.bfloat16).double()
+    else:
+        x, w, scale, b = _operands(rows, reduction, cols, seed=rows + cols, bias=direction == "bias")
+        got = quant_kernels.int8_linear_forward(x, w, scale, b, path="strip")
+        again = quant_kernels.int8_linear_forward(x, w, scale, b, path="strip")
+        decoded = quant_kernels.decode(w, scale, torch.bfloat16).double().t()
+    assert got.shape == (rows, cols)
+    assert torch.equal(got.view(torch.int16), again.view(torch.int16))
+    exact = x.double() @ decoded
+    if b is not None:
+        exact = exact + b.double()
+    _within_accumulation_bound(got, exact, x.double().abs() @ decoded.abs(), reduction)
+
+
+@pytest.mark.parametrize("rows,features", [(128, 64), (3136, 3136), (1040, 448)])
+def test_strip_reproduces_the_decoded_weight_bitwise(rows, features) -> None:
+    """One-hot operands: each output is one product plus zeros, whatever the split."""
+
+    eye = torch.eye(features, dtype=torch.bfloat16, device=DEV)
+    _, w, scale, _ = _operands(1, features, rows, seed=rows)
+    decoded = quant_kernels.decode(w, scale, torch.bfloat16)
+    y = quant_kernels.int8_linear_forward(eye, w, scale, path="strip")
+    assert torch.equal(y.view(torch.int16), decoded.t().contiguous().view(torch.int16))
+    _, w, scale, _ = _operands(1, rows, features, seed=rows + 1)
+    dx = quant_kernels.int8_linear_backward(eye, w, scale, torch.Size((features, rows)), path="strip")
+    assert torch.equal(dx.view(torch.int16), quant_kernels.decode(w, scale, torch.bfloat16).view(torch.int16))
+
+
+def test_unsplit_strip_adds_in_the_order_of_the_other_tiles() -> None:
+    # 2047 x 4096 from 704: one K group, no split; the fused path runs the small tile
+    x, w, scale, _ = _operands(2047, 704, 4096, seed=3)
+    assert torch.equal(quant_kernels.int8_linear_forward(x, w, scale, path="strip").view(torch.int16),
+                       quant_kernels.int8_linear_forward(x, w, scale, path="fused").view(torch.int16))
+    _, w, scale, _ = _operands(1, 4096, 704, seed=4)
+    shape = torch.Size((2047, 4096))
+    assert torch.equal(quant_kernels.int8_linear_backward(x, w, scale, shape, path="strip").view(torch.int16),
+                       quant_kernels.int8_linear_backward(x, w, scale, shape, path="fused").view(torch.int16))
+
+
+def test_strip_refuses_what_it_cannot_run() -> None:
+    x, w, scale, _ = _operands(64, 80, 64, seed=5)  # a reduction of 80
+    with pytest.raises(_native.EngineError, match="multiples of 64"):
+        quant_kernels.int8_linear_forward(x, w, scale, path="strip")
+    lib = _native.load()
+    x, w, scale, _ = _operands(33, 3072, 1040, seed=6)
+    y = torch.empty(33, 1040, dtype=torch.bfloat16, device=DEV)
+    need = lib.mo_int8_strip_workspace_bytes(33, 1040, 3072)
+    assert need >= 2 * 33 * 1040 * 4
+    work = torch.empty(need, dtype=torch.uint8, device=DEV)
+    stream = torch.cuda.current_stream(DEV).cuda_stream
+    rc = lib.mo_int8_strip_forward(x.data_ptr(), w.data_ptr(), scale.data_ptr(), 0, y.data_ptr(), 33, 3072, 1040,
+                                   work.data_ptr(), need - 256, stream)
+    assert rc == _native.MO_E_INVALID and b"workspace" in lib.mo_last_error()
+    # no workspace: the same product without a split
+    _native.check("mo_int8_strip_forward", lib.mo_int8_strip_forward(
+        x.data_ptr(), w.data_ptr(), scale.data_ptr(), 0, y.data_ptr(), 33, 3072, 1040, 0, 0, stream))
+    decoded = quant_kernels.decode(w, scale, torch.bfloat16).double().t()
+    _within_accumulation_bound(y, x.double() @ decoded, x.double().abs() @ decoded.abs(), 3072)
