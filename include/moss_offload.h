@@ -33,7 +33,7 @@
 extern "C" {
 #endif
 
-#define MO_ABI_VERSION 22
+#define MO_ABI_VERSION 23
 #define MO_MAX_DIMS 8
 
 /* Error codes outside the hipError_t range. */
@@ -459,6 +459,13 @@ int mo_streamer_reset_stats(mo_streamer* streamer);
  * instead of the fused kernels below. */
 int mo_int8_decode(uint64_t w, uint64_t scale, uint64_t out, uint32_t out_features, uint32_t in_features,
                    uint64_t stream);
+
+/* The same weight decoded transposed, `out` [in_features][out_features] bf16: the operand of an input
+ * gradient whose library GEMM reads the reduction (out_features) contiguously. Both features
+ * multiples of 16. No counterpart in the reference, whose eager path multiplies by the weight as
+ * decoded (quantization.py:54-65). */
+int mo_int8_decode_transposed(uint64_t w, uint64_t scale, uint64_t out, uint32_t out_features, uint32_t in_features,
+                              uint64_t stream);
 
 /* y[rows][out] = x[rows][in] . decode(w)^T (+ bias), on bf16 MFMA with fp32 accumulation, where
  * decode(w)[n][k] = bf16(w[n][k] * bf16(scale[n])), the decode of quant_kernels.py:126-131.

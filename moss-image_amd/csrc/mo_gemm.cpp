@@ -44,6 +44,7 @@ struct GemmModule {
   // [backward][small][tail]
   Kernel k[2][2][2];
   hipFunction_t decode = nullptr;     // mo_int8_decode_kernel
+  hipFunction_t decode_transposed = nullptr;
   hipFunction_t ws_fwd = nullptr;     // mo_int8_ws_fwd: weight in registers, column scales
   hipFunction_t ws_kscale = nullptr;  // mo_int8_ws_kscale: the same on a transposed weight, per-k scales
   hipFunction_t transpose = nullptr;  // mo_int8_transpose_kernel
@@ -103,6 +104,8 @@ int gemm_module(GemmModule* out) {
         }
     if ((e = hipModuleGetFunction(&m.decode, m.module, "mo_int8_decode_kernel")) != hipSuccess)
       return mo::set_hip_error((int)e, "hipModuleGetFunction (int8 decode)");
+    if ((e = hipModuleGetFunction(&m.decode_transposed, m.module, "mo_int8_decode_transposed_kernel")) != hipSuccess)
+      return mo::set_hip_error((int)e, "hipModuleGetFunction (int8 transposed decode)");
     if ((e = hipModuleGetFunction(&m.ws_fwd, m.module, "mo_int8_ws_fwd")) != hipSuccess ||
         (e = hipModuleGetFunction(&m.ws_kscale, m.module, "mo_int8_ws_kscale")) != hipSuccess ||
         (e = hipModuleGetFunction(&m.transpose, m.module, "mo_int8_transpose_kernel")) != hipSuccess ||
@@ -347,6 +350,23 @@ int strip_call(bool backward, uint64_t a, uint64_t w, uint64_t scale, uint64_t b
 }  // namespace
 
 extern "C" {
+
+int mo_int8_decode_transposed(uint64_t w, uint64_t scale, uint64_t out, uint32_t out_features, uint32_t in_features,
+                              uint64_t stream) {
+  if (int rc = check(w, w, scale, out, 1, in_features, out_features)) return rc;
+  GemmModule m;
+  if (int rc = gemm_module(&m)) return rc;
+  const void* q = (const void*)w;
+  const void* sc = (const void*)scale;
+  void* o = (void*)out;
+  uint32_t rows = out_features, cols = in_features;
+  void* params[] = {&q, &sc, &o, &rows, &cols};
+  const uint32_t blocks = ((rows + 127) / 128) * ((cols + 127) / 128);
+  const hipError_t e = hipModuleLaunchKernel(m.decode_transposed, blocks, 1, 1, 256, 1, 1, 0, (hipStream_t)stream,
+                                             params, nullptr);
+  if (e != hipSuccess) return mo::set_hip_error((int)e, "int8 transposed decode launch");
+  return 0;
+}
 
 int mo_int8_decode(uint64_t w, uint64_t scale, uint64_t out, uint32_t out_features, uint32_t in_features,
                    uint64_t stream) {

@@ -15,7 +15,7 @@ import torch  # noqa: F401  (must be imported before the library, see module doc
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libmoss_offload.so"
 
-MO_ABI_VERSION = 22
+MO_ABI_VERSION = 23
 MO_MAX_DIMS = 8
 
 MO_E_INVALID = 1001
@@ -250,6 +250,7 @@ SIGNATURES: dict[str, tuple] = {
     "mo_gradacc_get_stats": (ctypes.c_int, [ctypes.c_void_p, _P(MoGradaccStats)]),
     "mo_gradacc_reset_stats": (ctypes.c_int, [ctypes.c_void_p]),
     "mo_int8_decode": (ctypes.c_int, [_u64, _u64, _u64, ctypes.c_uint32, ctypes.c_uint32, _u64]),
+    "mo_int8_decode_transposed": (ctypes.c_int, [_u64, _u64, _u64, ctypes.c_uint32, ctypes.c_uint32, _u64]),
     "mo_wire_capacity": (_u64, [_u64]),
     "mo_wire_encode": (ctypes.c_int, [_u64, _u64, _u64, _u64, _u64, _u64]),
     "mo_wire_decode": (ctypes.c_int, [_u64, _u64, _u64, _u64, _u64]),

@@ -125,7 +125,18 @@ STRIP_LONG_ROWS = 6144
 LIBRARY_ROWS = 2048
 LIBRARY_WEIGHT = 16 << 20
 LONG_REDUCTION = 4
-PATHS = ("auto", "fused", "library", "strip")
+# Input gradients left to the library decode the weight transposed (mo_int8_decode_transposed), so
+# that its GEMM reads both operands along the reduction. Library on the weight as stored / transposed,
+# decode included, us:
+#   rows                  3400      4608      5700      6400      8192      11000     14000     17792
+#   3072 from 3072       73/66     85/74   113/115   118/122   146/133   198/178   229/201   307/258
+#   12288 from 3072    235/206   312/271   422/363   399/350   501/430   704/654   841/749  1103/945
+# Not for reductions under TRANSPOSED_REDUCTION (6200 rows of 3072 from 1040: 65/77), nor for outputs
+# a power of two wide, where the library's kernel for it is erratic (8192 from 3072: 2800 rows
+# 135/197, 4000 rows 169/150, 5700 rows 280/326), nor for long reductions (3072 from 24576: 7800
+# rows 1483/1536, 8192 rows 1044/923, 8600 rows 1409/1487).
+TRANSPOSED_REDUCTION = 2048
+PATHS = ("auto", "fused", "library", "strip", "transposed")
 
 
 def decode_hip(weight: torch.Tensor, scale: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -139,11 +150,24 @@ def decode_hip(weight: torch.Tensor, scale: torch.Tensor, *, out: torch.Tensor |
     return out
 
 
+def decode_transposed_hip(weight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+    """``decode(weight, scale, bfloat16).t()``, contiguous, in one HIP pass, bit for bit."""
+
+    lib = _native.load()
+    out_features, in_features = weight.shape
+    out = torch.empty((in_features, out_features), dtype=torch.bfloat16, device=weight.device)
+    _native.check("mo_int8_decode_transposed", lib.mo_int8_decode_transposed(
+        weight.data_ptr(), scale.data_ptr(), out.data_ptr(), out_features, in_features, _stream(weight)))
+    return out
+
+
 def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: int, backward: bool) -> str:
-    """The path a call takes: ``strip``, ``library`` or ``fused``."""
+    """The path a call takes: ``strip``, ``library``, ``transposed`` or ``fused``."""
 
     if path not in PATHS:
         raise ValueError(f"path must be one of {PATHS}")
+    if path == "transposed" and not backward:
+        raise ValueError("the transposed path is the input gradient's")
     if path != "auto":
         return path
     long_reduction = reduction >= LONG_REDUCTION * width
@@ -151,7 +175,11 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
         return "strip"
     if rows < LIBRARY_ROWS and weight.numel() < LIBRARY_WEIGHT:
         return "fused"
-    return "fused" if long_reduction and _splits(rows, width, reduction, backward) else "library"
+    if long_reduction and _splits(rows, width, reduction, backward):
+        return "fused"
+    if backward and reduction >= TRANSPOSED_REDUCTION and not long_reduction and width & (width - 1):
+        return "transposed"
+    return "library"
 
 
 def _strips(rows: int, reduction: int, width: int, backward: bool, long_reduction: bool) -> bool:
@@ -238,13 +266,21 @@ def int8_linear_backward(gradient: torch.Tensor, weight: torch.Tensor, scale: to
                          input_shape: torch.Size, *, out: torch.Tensor | None = None,
                          path: str = "auto") -> torch.Tensor:
     """``gradient @ decode(weight)``: the input gradient of the frozen int8 linear (``path`` as in
-    ``int8_linear_forward``; ``strip`` needs ``out_features`` a multiple of 64)."""
+    ``int8_linear_forward``; ``strip`` needs ``out_features`` a multiple of 64; ``transposed``: the
+    library GEMM on ``decode_transposed_hip``'s weight)."""
 
     lib = _native.load()
     matrix = gradient.reshape(-1, gradient.shape[-1]).to(torch.bfloat16).contiguous()
     rows, out_features = matrix.shape
     in_features = weight.shape[1]
     route = _route(path, rows, weight, out_features, in_features, True)
+    if route == "transposed":
+        decoded = decode_transposed_hip(weight, scale)
+        if out is None:
+            return F.linear(matrix, decoded).reshape(input_shape)
+        out = _output(out, (rows, in_features), gradient.device, "input-gradient")
+        torch.mm(matrix, decoded.t(), out=out)
+        return out.reshape(input_shape)
     if route == "library":
         if out is None:  # the eager path's call (see int8_linear_forward)
             return matrix.matmul(decode_hip(weight, scale)).reshape(input_shape)

@@ -68,6 +68,34 @@ def test_unsplit_strip_adds_in_the_order_of_the_other_tiles() -> None:
                        quant_kernels.int8_linear_backward(x, w, scale, shape, path="fused").view(torch.int16))
 
 
+@pytest.mark.parametrize("out_f,in_f", [(16, 16), (48, 80), (144, 272), (4112, 16), (3072, 1040)])
+def test_transposed_decode_matches_the_decode_bitwise(out_f, in_f) -> None:
+    _, w, scale, _ = _operands(1, in_f, out_f, seed=out_f + in_f)
+    scale[::7] = -scale[::7]
+    scale[::11] = 1.0 + 2.0**-8  # halfway between two bf16 values
+    got = quant_kernels.decode_transposed_hip(w, scale)
+    want = quant_kernels.decode(w, scale, torch.bfloat16).t().contiguous()
+    assert got.shape == (in_f, out_f) and torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_input_gradients_above_the_strips_take_the_transposed_weight() -> None:
+    rows, in_f, out_f = 4608, 1104, 2048
+    _, w, scale, _ = _operands(1, in_f, out_f, seed=8)
+    dy = _operands(rows, out_f, 16, seed=9)[0]
+    shape = torch.Size((rows, in_f))
+    got = quant_kernels.int8_linear_backward(dy, w, scale, shape)
+    named = quant_kernels.int8_linear_backward(dy, w, scale, shape, path="transposed")
+    assert torch.equal(got.view(torch.int16), named.view(torch.int16))
+    buf = torch.empty(rows * in_f, dtype=torch.bfloat16, device=DEV)
+    out = quant_kernels.int8_linear_backward(dy, w, scale, shape, out=buf)
+    assert out.data_ptr() == buf.data_ptr()
+    decoded = quant_kernels.decode(w, scale, torch.bfloat16).double()
+    for y in (got, out):
+        _within_accumulation_bound(y, dy.double() @ decoded, dy.double().abs() @ decoded.abs(), out_f)
+    with pytest.raises(ValueError, match="input gradient"):
+        quant_kernels.int8_linear_forward(dy, w.t().contiguous(), scale[:in_f], path="transposed")
+
+
 def test_strip_refuses_what_it_cannot_run() -> None:
     x, w, scale, _ = _operands(64, 80, 64, seed=5)  # a reduction of 80
     with pytest.raises(_native.EngineError, match="multiples of 64"):
