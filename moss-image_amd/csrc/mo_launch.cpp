@@ -330,8 +330,8 @@ int wire_encode(uint64_t raw, uint64_t raw_bytes, uint64_t wire, uint64_t capaci
   }
   if (tiles) {
     void* params[] = {&r, &n, &w, &cap};
-    if ((e = hipModuleLaunchKernel(m.wire_encode, groups, 1, 1, kThreads, 1, 1, 0, stream, params,
-                                   nullptr)) != hipSuccess)
+    if ((e = hipModuleLaunchKernel(m.wire_encode, (uint32_t)tiles, 1, 1, kThreads, 1, 1, 0, stream, params,
+                                   nullptr)) != hipSuccess)  // one workgroup per tile
       return (int)e;
   }
   return 0;

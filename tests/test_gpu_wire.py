@@ -126,6 +126,42 @@ def test_large_gaussian_buffer_round_trip_and_ratio() -> None:
     assert torch.equal(out.view(torch.int16), src.view(torch.int16))
 
 
+@pytest.mark.parametrize("tiles,distinct", [(4097, 3), (4096, 40), (33, 256), (5, 1)])
+def test_tile_counts_and_alphabets_round_trip(tiles, distinct) -> None:
+    """Tile counts at the edge of the offset scan's chunk (4 096 tiles, 128 MiB) and past it, and
+    tables of 1, a few and all 256 exponents (the kernel's table, state and stream copies start at
+    every 4-byte position of those sizes): the tile offsets rise by whole 16-byte pieces to the
+    coded size, and the round trip is bitwise."""
+
+    lib = _native.load()
+    stream = torch.cuda.current_stream(DEV).cuda_stream
+    words = tiles * 16384
+    g = torch.Generator(device=DEV).manual_seed(tiles)
+    # exponents skewed to the small ones, so that a tile of all 256 is coded, not stored raw
+    u = torch.rand(words, device=DEV, generator=g)
+    e = (u * u * u * u * distinct).to(torch.int32).clamp_(max=distinct - 1)
+    e[:: words // max(words // 64, 1)] = torch.arange(distinct, device=DEV, dtype=torch.int32).repeat(
+        (words // 64 + distinct) // distinct)[: words // 64]
+    sm = torch.randint(0, 256, (words,), device=DEV, generator=g, dtype=torch.int32)
+    raw = (((sm & 0x80) << 8) | (e << 7) | (sm & 0x7F)).to(torch.int16)
+    nbytes = 2 * words
+    cap = lib.mo_wire_capacity(nbytes)
+    wire = torch.empty(cap, dtype=torch.uint8, device=DEV)
+    total = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+    _native.check("mo_wire_encode", lib.mo_wire_encode(raw.data_ptr(), nbytes, wire.data_ptr(), cap, total.data_ptr(),
+                                                       stream))
+    torch.cuda.synchronize()
+    coded = int(total[0])
+    assert coded < 0.95 * nbytes
+    offsets = wire[16:16 + 4 * tiles].cpu().view(torch.int32).to(torch.int64)
+    sizes = torch.diff(torch.cat([offsets, torch.tensor([coded])]))
+    assert bool((sizes > 16384).all()) and bool((sizes <= 32768 + 16).all()) and bool((offsets % 16 == 0).all())
+    out = torch.zeros_like(raw)
+    _native.check("mo_wire_decode", lib.mo_wire_decode(wire.data_ptr(), coded, out.data_ptr(), nbytes, stream))
+    torch.cuda.synchronize()
+    assert torch.equal(out, raw)
+
+
 def test_rejects_short_wire_buffer_and_misalignment() -> None:
     lib = _native.load()
     stream = torch.cuda.current_stream(DEV).cuda_stream
