@@ -790,32 +790,39 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_wire_encode_kernel
   }
 }
 
-// Decode a coded stream of `raw_bytes` into `raw`. Grid: max(ceil(tiles / 4), 1) workgroups, one
-// wave per tile; the first workgroup also copies the raw tail. 6.5 KiB of LDS a wave: the table
-// entries by rank, each slot's rank, a ring of the stream's next 512 words, and one group's
-// exponents: state l decodes the tile's words 64 j + l, so the exponents of 8 rounds are 1 KiB of
-// consecutive words, written out as one 16-byte store a lane. Reads go through
-// a resource over [wire, wire + wire_bytes), and writes stay inside [raw, raw + raw_bytes)
-// whatever the stream holds: a damaged header is clamped, and table values only index the
-// wave's own LDS arrays.
-extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_wire_decode_kernel(const char* wire, uint64_t wire_bytes,
-                                                                                  uint64_t raw_bytes, char* raw) {
+// Decode a coded stream of `raw_bytes` into `raw`. Grid: max(tiles, 1) workgroups of one wave, a tile
+// each; the first also copies the raw tail. 8 KiB of LDS: each slot's rank, the table entries by
+// rank, a ring of the stream's next 512 words, and one group's exponents: state l decodes the
+// tile's words 64 j + l, so the exponents of 8 rounds are 1 KiB of consecutive words, written out
+// as one 16-byte store a lane.
+// Bound by a round's chain of three LDS reads (slot, entry, stream word) and the vector instructions
+// between them, and with 13.5 waves a CU (113 MB) nearly as much by the issue of those: so a round
+// is kept short. A wave is its own workgroup (its arrays lie at fixed LDS addresses; 13.5 waves a
+// CU also spread better than 3.4 groups of four); an entry's parts sit where the multiply, the
+// subtraction and the byte store take them as they are; the ring repeats its first 256 words past
+// its end, so that the four rounds between refills index it without wrapping; and a byte select
+// brings a stream word in. 113 MB: 67 us with four
+// tiles a workgroup and 26 instructions a round, now 53.5; a 256 KiB segment 48, now 33.
+// Reads go through a resource over [wire, wire + wire_bytes), and writes stay inside
+// [raw, raw + raw_bytes) whatever the stream holds: a damaged header is clamped, and table values
+// only index the wave's own LDS arrays.
+extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const char* wire, uint64_t wire_bytes,
+                                                                       uint64_t raw_bytes, char* raw) {
   using namespace mo;
-  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-  constexpr uint32_t kSlots = 1u << kWireProbBits, kRing = 512;
-  __shared__ __attribute__((aligned(16))) unsigned char slot_rank[kWireWaves][kSlots];
-  __shared__ uint32_t ranks[kWireWaves][256];  // table entry -> exponent | (f - 1) << 8 | c << 20
-  __shared__ __attribute__((aligned(16))) unsigned short rings[kWireWaves][kRing];
-  __shared__ __attribute__((aligned(16))) unsigned char groups[kWireWaves][8 * kWireLanes];
-  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr uint32_t kSlots = 1u << kWireProbBits, kRing = 512, kAgain = 256;
+  __shared__ __attribute__((aligned(16))) unsigned char slot_rank[kSlots];
+  __shared__ __attribute__((aligned(16))) mo_u32x2 rank_entry[256];  // {f, c | exponent << 16}
+  __shared__ __attribute__((aligned(16))) unsigned short ring[kRing + kAgain];
+  __shared__ __attribute__((aligned(16))) unsigned char group[8 * kWireLanes];
+  const uint32_t lane = threadIdx.x;
   const __amdgpu_buffer_rsrc_t w = wire_rsrc(wire, wire_bytes);
   if (blockIdx.x == 0) {
     const uint64_t tail = raw_bytes % kWireBlockBytes, tail_dst = wire_blocks(raw_bytes) * kWireBlockBytes;
     const uint64_t data_start = wire_data_start(raw_bytes);
-    for (uint64_t i = threadIdx.x; i < tail; i += kThreads)
+    for (uint64_t i = lane; i < tail; i += 64)
       st<kG>(raw + tail_dst + i, (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(w, (int)(data_start + i), 0, 0));
   }
-  const uint64_t tile = (uint64_t)blockIdx.x * kWireTilesPerGroup + wave;
+  const uint64_t tile = blockIdx.x;
   if (tile >= wire_tiles(raw_bytes)) return;
   const uint32_t n = wire_tile_words(raw_bytes, tile), J = n / kWireLanes;
   char* const dst = raw + tile * kWireTileRaw;
@@ -830,13 +837,14 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_wire_decode_kernel
     return;
   }
   const uint32_t nsym = min((head >> 8) & 0x1ffu, 256u);
-  MO_LDS unsigned char* const sr = (MO_LDS unsigned char*)slot_rank[wave];
-  MO_LDS uint32_t* const rk = (MO_LDS uint32_t*)ranks[wave];
-  MO_LDS unsigned short* const ring = (MO_LDS unsigned short*)rings[wave];
+  MO_LDS unsigned char* const sr = (MO_LDS unsigned char*)slot_rank;
+  MO_LDS mo_u32x2* const re = (MO_LDS mo_u32x2*)rank_entry;
+  MO_LDS unsigned short* const words = (MO_LDS unsigned short*)ring;
+  MO_LDS unsigned char* const grp = (MO_LDS unsigned char*)group;
   // Table entries in rank order with their cumulative frequencies; each entry's first slot is
   // marked with its rank (rank 0 starts at slot 0, where every slot's mark starts).
   const uint32_t tab = body + n;
-  for (uint32_t i = lane; i < kSlots / 4; i += 64) *(MO_LDS uint32_t*)(sr + 4 * i) = 0;
+  for (uint32_t i = lane; i < kSlots / 16; i += 64) *(MO_LDS mo_u32x4*)(sr + 16 * i) = mo_u32x4{0, 0, 0, 0};
   wave_lds_fence();
   uint32_t carry = 0;
 #pragma unroll
@@ -846,70 +854,88 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_wire_decode_kernel
     const uint32_t f = r < nsym ? min((e >> 8) & 0x1fffu, kSlots) : 0u;
     const uint32_t incl = wave_scan(f, lane), c = carry + incl - f;
     carry += (uint32_t)__shfl((int)incl, 63, 64);
-    rk[r] = (e & 0xffu) | (((f - 1) & 0xfffu) << 8) | ((c & 0xfffu) << 20);
+    re[r] = mo_u32x2{f, (c & 0xffffu) | ((e & 0xffu) << 16)};
     if (f && c < kSlots) sr[c] = (unsigned char)r;
   }
   wave_lds_fence();
-  // Every slot's rank: the last mark at or before it (marks rise with the slot), 64 slots a
-  // round as a prefix maximum over the round's lanes and the rounds before.
+  // Every slot's rank: the last mark at or before it (marks rise with the slot). Four consecutive
+  // slots a lane: the byte maxima within its word, a prefix maximum over the lanes' last bytes, and
+  // the carry of the rounds before.
   uint32_t before = 0;
-  for (uint32_t row = 0; row < kSlots / 64; ++row) {
-    const uint32_t slot = 64 * row + lane;
-    const uint32_t cur = max(before, wave_scan_max_dpp(sr[slot]));
-    before = (uint32_t)__builtin_amdgcn_readlane((int)cur, 63);
-    sr[slot] = (unsigned char)cur;
+  for (uint32_t row = 0; row < kSlots / 256; ++row) {
+    const uint32_t four = *(const MO_LDS uint32_t*)(sr + 256 * row + 4 * lane);
+    uint32_t m[4];
+    m[0] = four & 0xffu;
+#pragma unroll
+    for (int k = 1; k < 4; ++k) m[k] = max(m[k - 1], (four >> (8 * k)) & 0xffu);
+    const uint32_t upto = wave_scan_max_dpp(m[3]);
+    const uint32_t left = max(before, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x138, 0xf, 0xf, false));  // wave_shr:1
+    *(MO_LDS uint32_t*)(sr + 256 * row + 4 * lane) =
+        max(left, m[0]) | (max(left, m[1]) << 8) | (max(left, m[2]) << 16) | (max(left, m[3]) << 24);
+    before = max(before, (uint32_t)__builtin_amdgcn_readlane((int)upto, 63));
   }
-  // States, and the stream's first 512 words into the ring (word i at i % 512); `next` holds
-  // the 2 words this lane brings in at the next refill.
+  // States, and the stream's first 512 words into the ring (word i at i % 512, and again at
+  // 512 + i % 512 where that is below 768); `next` holds the 2 words this lane brings in at the
+  // next refill.
   const uint32_t states = tab + (uint32_t)wire_align16(4 * nsym);
   uint32_t x = __builtin_amdgcn_raw_buffer_load_b32(w, (int)(states + 4 * lane), 0, 0);
   const uint32_t stream = states + 4 * kWireLanes;
+  auto refill = [&](uint32_t at, uint32_t v) {  // 128 words from ring word `at` on, a multiple of 128
+    *(MO_LDS uint32_t*)(words + at + 2 * lane) = v;
+    if (at < kAgain) *(MO_LDS uint32_t*)(words + kRing + at + 2 * lane) = v;
+  };
 #pragma unroll
   for (uint32_t q = 0; q < 4; ++q)
-    *(MO_LDS uint32_t*)(ring + 128 * q + 2 * lane) =
-        __builtin_amdgcn_raw_buffer_load_b32(w, (int)(stream + 256 * q + 4 * lane), 0, 0);
+    refill(128 * q, __builtin_amdgcn_raw_buffer_load_b32(w, (int)(stream + 256 * q + 4 * lane), 0, 0));
   uint32_t next = __builtin_amdgcn_raw_buffer_load_b32(w, (int)(stream + 1024 + 4 * lane), 0, 0);
   wave_lds_fence();
   uint32_t ptr = 0, wb = 0;  // words read so far; the first word the ring still holds
   // the group's sign-mantissa bytes (words 8 l .. 8 l + 7 of its 512), one group ahead
-  MO_LDS unsigned char* const grp = (MO_LDS unsigned char*)groups[wave];
   const uint32_t ngroups = J / 8;
-  u32x2 sm_next = __builtin_amdgcn_raw_buffer_load_b64(w, (int)(body + 8 * lane), 0, 0);
+  mo_u32x2 sm_next = __builtin_amdgcn_raw_buffer_load_b64(w, (int)(body + 8 * lane), 0, 0);
   for (uint32_t g = 0; g < ngroups; ++g) {
-    const u32x2 sm = sm_next;
+    const mo_u32x2 sm = sm_next;
     sm_next = __builtin_amdgcn_raw_buffer_load_b64(w, (int)(body + 512 * (g + 1) + 8 * lane), 0, 0);  // a spare past the last
+    uint32_t at;  // the ring's byte at which the next word lies
+    auto wrap = [&] {
+      at = 2 * (ptr % kRing);
+      asm("" : "+s"(at));  // a number of its own: known to be a double, it is doubled again each round
+    };
+    wrap();
 #pragma unroll
     for (uint32_t r = 0; r < 8; ++r) {
-      const uint32_t slot = x & (kSlots - 1);
-      const uint32_t t = rk[sr[slot]];
-      x = (((t >> 8) & 0xfffu) + 1) * (x >> kWireProbBits) + slot - (t >> 20);
+      const uint32_t slot = x % kSlots;
+      const mo_u32x2 t = re[sr[slot]];
+      const uint32_t f = t[0], ce = t[1];
+      x = __umul24(f, x >> kWireProbBits) + (slot - (ce & 0xffffu));
       const bool need = x < kWireStateLow;
       const uint64_t bal = __ballot(need);
-      const uint32_t word = ring[(ptr + lanes_below(bal)) & (kRing - 1)];
-      x = need ? (x << 16) | word : x;
+      const uint32_t mine = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+      const uint32_t word = *(const MO_LDS unsigned short*)((const MO_LDS unsigned char*)words + (2 * mine + at));
+      x = __builtin_amdgcn_perm(x, word, need ? 0x05040100u : 0x07060504u);  // (x << 16) | word, or x
       ptr += (uint32_t)__popcll(bal);
-      grp[64 * r + lane] = (unsigned char)t;
-      if (ptr - wb >= 128) {
-        // words [wb, wb + 128) are consumed: their ring quarter takes words [wb + 512, wb + 640)
-        *(MO_LDS uint32_t*)(ring + (wb & (kRing - 1)) + 2 * lane) = next;
-        wb += 128;
-        next = __builtin_amdgcn_raw_buffer_load_b32(w, (int)(stream + 2 * (wb + kRing) + 4 * lane), 0, 0);
-        wave_lds_fence();
+      at += 2 * (uint32_t)__popcll(bal);
+      grp[64 * r + lane] = (unsigned char)(ce >> 16);
+      // Every four rounds, which read at most 256 words: the ring holds at least 512 - 127 of them.
+      // Words [wb, wb + 128) are consumed: their ring quarter takes words [wb + 512, wb + 640).
+      if (r % 4 == 3) {
+        while (ptr - wb >= 128) {
+          refill(wb % kRing, next);
+          wb += 128;
+          next = __builtin_amdgcn_raw_buffer_load_b32(w, (int)(stream + 2 * (wb + kRing) + 4 * lane), 0, 0);
+          wave_lds_fence();
+        }
+        wrap();
       }
     }
     wave_lds_fence();
-    const u32x2 ex = *(const MO_LDS u32x2*)(grp + 8 * lane);
+    const mo_u32x2 ex = *(const MO_LDS mo_u32x2*)(grp + 8 * lane);
     uint32_t o[4];
 #pragma unroll
-    for (uint32_t k = 0; k < 8; k += 2) {
-      uint32_t pair = 0;
-#pragma unroll
-      for (uint32_t h = 0; h < 2; ++h) {
-        const uint32_t i = k + h;
-        const uint32_t s = (sm[i >> 2] >> (8 * (i & 3))) & 0xffu, e = (ex[i >> 2] >> (8 * (i & 3))) & 0xffu;
-        pair |= (((s & 0x80u) << 8) | (e << 7) | (s & 0x7fu)) << (16 * h);
-      }
-      o[k >> 1] = pair;
+    for (uint32_t k = 0; k < 4; ++k) {  // words 2k and 2k + 1: their bytes spread to the halves, then shifted into place
+      const uint32_t spread = k & 1 ? 0x0c070c06u : 0x0c050c04u;
+      const uint32_t s = __builtin_amdgcn_perm(sm[k >> 1], 0u, spread), m = __builtin_amdgcn_perm(ex[k >> 1], 0u, spread);
+      o[k] = ((s & 0x00800080u) << 8) | (m << 7) | (s & 0x007f007fu);
     }
     st16(dst + 1024 * (uint64_t)g + 16 * lane, make_uint4(o[0], o[1], o[2], o[3]));
     wave_lds_fence();  // the group buffer is read before the next group writes it

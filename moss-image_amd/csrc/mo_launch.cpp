@@ -345,9 +345,8 @@ int wire_decode(uint64_t wire, uint64_t wire_bytes, uint64_t raw, uint64_t raw_b
   void* r = (void*)raw;
   uint64_t wb = wire_bytes, n = raw_bytes;
   void* params[] = {&w, &wb, &n, &r};
-  const uint32_t groups = (uint32_t)((tiles + kWireTilesPerGroup - 1) / kWireTilesPerGroup);  // one wave per tile
-  return (int)hipModuleLaunchKernel(m.wire_decode, groups ? groups : 1, 1, 1, kThreads, 1, 1, 0, stream,
-                                    params, nullptr);
+  return (int)hipModuleLaunchKernel(m.wire_decode, tiles ? (uint32_t)tiles : 1, 1, 1, kWireLanes, 1, 1, 0, stream,
+                                    params, nullptr);  // a wave per tile
 }
 
 }  // namespace mo
