@@ -10,10 +10,12 @@
 //           per lane, no index arithmetic.
 //   RUNS    contiguous runs whose length, start and strides are multiples of 16 B: each
 //           16-byte chunk is located with fast division over the canonical dimensions.
-//   ELEM    anything else (misaligned bases, odd run lengths, element-strided innermost
-//           dimension): elements are gathered one by one into LDS and the tile is written
-//           to the payload with 128-bit stores (pack), or read from the payload with 128-bit
-//           loads into LDS and scattered from there (unpack).
+//   ROWS    contiguous runs off that grid (misaligned bases, odd run lengths or strides): each
+//           16-byte payload chunk is one unaligned 128-bit access of its run; a chunk that
+//           crosses into the next run moves element by element.
+//   ELEM    an element-strided innermost dimension: elements are gathered one by one into LDS
+//           and the tile is written to the payload with 128-bit stores (pack), or read from the
+//           payload with 128-bit loads into LDS and scattered from there (unpack).
 //   NARROW  a contiguous float32 tensor whose values are exactly bfloat16: the payload holds
 //           the high 16 bits of each element (pack reads 32 B and writes 16 B a chunk; unpack
 //           writes the halves back with zero low bits), so the same bits cross the host link
@@ -44,7 +46,7 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t n, uint32_t m, uint32_t s) {
 }
 
 // Address offset (bytes, relative to the tensor base) of unit `u` of a piece's tensor side.
-// A unit is a 16-byte chunk (RUNS) or an element (ELEM).
+// A unit is a 16-byte chunk (RUNS) or an element (ROWS, ELEM).
 __device__ __forceinline__ uint64_t unit_offset(const KDesc& d, uint32_t u) {
   uint32_t q = fdiv(u, d.inner.m, d.inner.s);
   uint64_t off = (uint64_t)(u - q * d.inner.d) * d.inner_stride;
@@ -62,59 +64,45 @@ __device__ __forceinline__ uint64_t unit_offset(const KDesc& d, uint32_t u) {
 
 // Every device pointer reaches the kernels as an integer inside a descriptor, so the compiler
 // cannot infer its address space and would emit flat (generic) memory instructions. The
-// accessors below name the space: global (HBM or pinned host memory) or LDS.
+// accessors below name the space: global (HBM or pinned host memory).
 #define MO_GLOBAL __attribute__((address_space(1)))
 #define MO_LDS __attribute__((address_space(3)))
-
-enum Space { kG, kL };
 
 // 16-byte values move as a native vector: uint4 is a class whose copy constructor takes a
 // generic reference, which would turn the access back into a flat one.
 typedef unsigned int mo_u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int mo_u32x2 __attribute__((ext_vector_type(2)));
 
-template <Space S, typename T>
+template <typename T>
 __device__ __forceinline__ T ld(const char* p) {
-  if (S == kG) return *(const MO_GLOBAL T*)p;
-  return *(const MO_LDS T*)p;
+  return *(const MO_GLOBAL T*)p;
 }
-template <Space S, typename T>
+template <typename T>
 __device__ __forceinline__ void st(char* p, T v) {
-  if (S == kG) *(MO_GLOBAL T*)p = v;
-  else *(MO_LDS T*)p = v;
+  *(MO_GLOBAL T*)p = v;
 }
 template <>
-__device__ __forceinline__ uint4 ld<kG, uint4>(const char* p) {
+__device__ __forceinline__ uint4 ld<uint4>(const char* p) {
   const mo_u32x4 x = *(const MO_GLOBAL mo_u32x4*)p;
   return make_uint4(x.x, x.y, x.z, x.w);
 }
 template <>
-__device__ __forceinline__ uint4 ld<kL, uint4>(const char* p) {
-  const mo_u32x4 x = *(const MO_LDS mo_u32x4*)p;
-  return make_uint4(x.x, x.y, x.z, x.w);
-}
-template <>
-__device__ __forceinline__ void st<kG, uint4>(char* p, uint4 v) {
+__device__ __forceinline__ void st<uint4>(char* p, uint4 v) {
   *(MO_GLOBAL mo_u32x4*)p = mo_u32x4{v.x, v.y, v.z, v.w};
 }
-template <>
-__device__ __forceinline__ void st<kL, uint4>(char* p, uint4 v) {
-  *(MO_LDS mo_u32x4*)p = mo_u32x4{v.x, v.y, v.z, v.w};
-}
 
-template <Space D, Space S>
 __device__ __forceinline__ void copy_elem(char* dst, const char* src, uint32_t eb) {
   switch (eb) {
-    case 1: st<D>(dst, ld<S, uint8_t>(src)); break;
-    case 2: st<D>(dst, ld<S, uint16_t>(src)); break;
-    case 4: st<D>(dst, ld<S, uint32_t>(src)); break;
-    case 8: st<D>(dst, ld<S, uint64_t>(src)); break;
-    default: st<D>(dst, ld<S, uint4>(src)); break;
+    case 1: st(dst, ld<uint8_t>(src)); break;
+    case 2: st(dst, ld<uint16_t>(src)); break;
+    case 4: st(dst, ld<uint32_t>(src)); break;
+    case 8: st(dst, ld<uint64_t>(src)); break;
+    default: st(dst, ld<uint4>(src)); break;
   }
 }
 
-__device__ __forceinline__ uint4 ld16(const char* p) { return ld<kG, uint4>(p); }
-__device__ __forceinline__ void st16(char* p, uint4 v) { st<kG>(p, v); }
+__device__ __forceinline__ uint4 ld16(const char* p) { return ld<uint4>(p); }
+__device__ __forceinline__ void st16(char* p, uint4 v) { st(p, v); }
 
 // Streaming store for the staging payload: it is written once and next read by a DMA engine,
 // so the write is marked non-temporal (no reuse expected in the GPU caches).
@@ -193,13 +181,175 @@ __device__ __forceinline__ void narrow_chunk(char* payload16, char* tensor32) {
   }
 }
 
+// `body` with a value of the element type of `eb` bytes.
+template <typename F>
+__device__ __forceinline__ void with_element(uint32_t eb, F&& body) {
+  switch (eb) {
+    case 1: body(uint8_t()); break;
+    case 2: body(uint16_t()); break;
+    case 4: body(uint32_t()); break;
+    case 8: body(uint64_t()); break;
+    default: body(mo_u32x4{0, 0, 0, 0}); break;
+  }
+}
+
+// 16 bytes at any byte address (global accesses of any alignment are one instruction under the
+// unaligned access mode every HSA kernel runs in).
+typedef unsigned int mo_u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+
+// Address offsets of the units u[0 .. N - 1], and the units of their innermost runs from them on:
+// unit_offset with the dimensions outermost, so that N chains run side by side in little code.
+template <int N>
+__device__ __forceinline__ void unit_offsets(const KDesc& d, const uint32_t (&u)[N], uint64_t (&off)[N], uint32_t (&left)[N]) {
+  uint32_t q[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    q[i] = fdiv(u[i], d.inner.m, d.inner.s);
+    const uint32_t at = u[i] - q[i] * d.inner.d;
+    off[i] = (uint64_t)at * d.inner_stride;
+    left[i] = d.inner.d - at;
+  }
+#pragma unroll 1
+  for (uint32_t k = 0; k < d.nouter; ++k) {
+    const KFastDiv f = d.outer[k];
+    const uint64_t stride = d.ostride[k];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const uint32_t q2 = fdiv(q[i], f.m, f.s);
+      off[i] += (uint64_t)(q[i] - q2 * f.d) * stride;
+      q[i] = q2;
+    }
+  }
+}
+
+// The 16 payload bytes of chunk `c`, whose elements cross from one run into the next (runs hold at
+// least 16 bytes): `n0` elements at `t0`, the others at `t1`, all in flight together.
+template <bool kPack, typename T>
+__device__ __forceinline__ void split_chunk(char* payload16, char* t0, char* t1, uint32_t n0) {
+  constexpr uint32_t kPer = 16 / sizeof(T);
+  union {
+    mo_u32x4 v;
+    T e[kPer];
+  } x;
+  if (!kPack) x.v = *(const MO_GLOBAL mo_u32x4*)payload16;
+  char* const second = t1 - (uint64_t)n0 * sizeof(T);
+#pragma unroll
+  for (uint32_t j = 0; j < kPer; ++j) {
+    char* const at = (j < n0 ? t0 : second) + j * sizeof(T);
+    if (kPack) x.e[j] = *(const MO_GLOBAL T*)at;
+    else *(MO_GLOBAL T*)at = x.e[j];
+  }
+  if (kPack) __builtin_nontemporal_store(x.v, (MO_GLOBAL mo_u32x4*)payload16);
+}
+
+// ROWS: one tile of contiguous runs off the 16-byte grid. Every lane locates its kUnroll chunks of
+// 16 payload bytes and has them in flight together; chunks that cross into the next run follow.
+// Memory-bound where runs are long; taken element by element, such a tile was bound by its
+// dependent round trips (32 a lane for 2-byte elements, 64 for bytes). Pack and unpack of 2 693 rows
+// of 6 144 bytes from an odd element on: 14.4 and 15.3 us, now 5.4 and 6.4 (6.2 and 5.2 TB/s); rows
+// of 67 bytes: 22.0 and 19.9, now 6.7 and 7.1.
 template <bool kPack>
-__device__ __forceinline__ void copy_tile_elem(const KDesc& d, uint64_t tile_off, uint32_t tile_bytes, char* payload,
-                                               char* tensor, uint32_t eb, uint32_t tid);
+__device__ __forceinline__ void rows_tile(const KDesc& d, uint32_t e0, uint32_t tile_bytes, char* payload, char* tensor,
+                                          uint32_t eb, uint32_t tid) {
+  const uint32_t nchunk = tile_bytes / 16, per = 16 / eb;
+  uint32_t e[kUnroll], left[kUnroll];
+  uint64_t off[kUnroll];
+  mo_u32x4 v[kUnroll];
+  bool split = false;
+#pragma unroll
+  for (int k = 0; k < kUnroll; ++k) e[k] = e0 + (k * kThreads + tid) * per;
+  unit_offsets(d, e, off, left);
+#pragma unroll
+  for (int k = 0; k < kUnroll; ++k) {
+    const uint32_t c = k * kThreads + tid;
+    if (c >= nchunk) continue;
+    if (left[k] < per) split = true;
+    else v[k] = kPack ? *(const MO_GLOBAL mo_u32x4_any*)(tensor + off[k]) : *(const MO_GLOBAL mo_u32x4*)(payload + 16 * (size_t)c);
+  }
+#pragma unroll
+  for (int k = 0; k < kUnroll; ++k) {
+    const uint32_t c = k * kThreads + tid;
+    if (c >= nchunk || left[k] < per) continue;
+    if (kPack) __builtin_nontemporal_store(v[k], (MO_GLOBAL mo_u32x4*)(payload + 16 * (size_t)c));
+    else *(MO_GLOBAL mo_u32x4_any*)(tensor + off[k]) = v[k];
+  }
+  if (__builtin_amdgcn_ballot_w64(split) != 0) {
+#pragma unroll 1
+    for (uint32_t c = tid; c < nchunk; c += kThreads) {
+      const uint32_t first = e0 + c * per;
+      const uint32_t n0 = d.inner.d - (first - fdiv(first, d.inner.m, d.inner.s) * d.inner.d);
+      if (n0 >= per) continue;
+      const uint32_t both[2] = {first, first + n0};
+      uint32_t unused[2];
+      uint64_t at[2];
+      unit_offsets(d, both, at, unused);
+      with_element(eb, [&](auto zero) {
+        split_chunk<kPack, decltype(zero)>(payload + 16 * (size_t)c, tensor + at[0], tensor + at[1], n0);
+      });
+    }
+  }
+  for (uint32_t b = nchunk * 16 + tid * eb; b < tile_bytes; b += kThreads * eb) {
+    char* const t = tensor + unit_offset(d, e0 + b / eb);
+    if (kPack) copy_elem(payload + b, t, eb);
+    else copy_elem(t, payload + b, eb);
+  }
+}
+
+// ELEM: one tile of a view whose innermost stride is not its element size (or whose runs are under
+// 16 bytes), staged in LDS. The payload side moves in 16-byte chunks; on the tensor side
+// consecutive lanes take consecutive elements, kInFlight of them a lane at a time (one at a time, a
+// tile was as many dependent round trips; more than four take registers from the other tiles of a
+// launch). Every other one of 2 693 x 256 halves: 11.3 and 10.4 us, now 6.9 and 5.1.
+template <bool kPack, typename T>
+__device__ __forceinline__ void elem_tile(const KDesc& d, uint32_t e0, uint32_t tile_bytes, char* payload, char* tensor,
+                                          uint32_t tid, MO_LDS char* lds) {
+  constexpr int kInFlight = 4;
+  const uint32_t nelem = tile_bytes / sizeof(T), nvec = tile_bytes / 16;
+  MO_LDS T* const el = (MO_LDS T*)lds;
+  MO_LDS mo_u32x4* const vec = (MO_LDS mo_u32x4*)lds;
+  if (!kPack) {
+    mo_u32x4 p[kUnroll];
+#pragma unroll
+    for (int k = 0; k < kUnroll; ++k) {
+      const uint32_t c = k * kThreads + tid;
+      if (c < nvec) p[k] = *(const MO_GLOBAL mo_u32x4*)(payload + 16 * (size_t)c);
+    }
+#pragma unroll
+    for (int k = 0; k < kUnroll; ++k)
+      if (k * kThreads + tid < nvec) vec[k * kThreads + tid] = p[k];
+    for (uint32_t j = nvec * 16 / sizeof(T) + tid; j < nelem; j += kThreads) el[j] = *(const MO_GLOBAL T*)(payload + j * sizeof(T));
+    __syncthreads();
+  }
+#pragma unroll 1
+  for (uint32_t j0 = tid; j0 < nelem; j0 += kThreads * kInFlight) {
+    T v[kInFlight];
+    uint32_t e[kInFlight], unused[kInFlight];
+    uint64_t off[kInFlight];
+#pragma unroll
+    for (int k = 0; k < kInFlight; ++k) e[k] = e0 + j0 + k * kThreads;
+    unit_offsets(d, e, off, unused);
+#pragma unroll
+    for (int k = 0; k < kInFlight; ++k) {
+      const uint32_t j = j0 + k * kThreads;
+      if (j >= nelem) continue;
+      if (kPack) v[k] = *(const MO_GLOBAL T*)(tensor + off[k]);
+      else *(MO_GLOBAL T*)(tensor + off[k]) = el[j];
+    }
+    if (!kPack) continue;
+#pragma unroll
+    for (int k = 0; k < kInFlight; ++k)
+      if (j0 + k * kThreads < nelem) el[j0 + k * kThreads] = v[k];
+  }
+  if (kPack) {
+    __syncthreads();
+    for (uint32_t c = tid; c < nvec; c += kThreads) __builtin_nontemporal_store(vec[c], (MO_GLOBAL mo_u32x4*)(payload + 16 * (size_t)c));
+    for (uint32_t j = nvec * 16 / sizeof(T) + tid; j < nelem; j += kThreads) *(MO_GLOBAL T*)(payload + j * sizeof(T)) = el[j];
+  }
+}
 
 // One 16 KiB tile (`tile`, numbered within the launch) of piece `d`. kElem: the launch may hold
-// ELEM pieces, whose LDS staging buffer every workgroup of the launch then reserves; launches
-// without them use the instantiation that reserves no LDS.
+// ROWS and ELEM pieces, for which every workgroup of the launch then reserves the LDS staging
+// buffer and more registers; launches without them use the instantiation without either.
 template <bool kPack, bool kElem>
 __device__ __forceinline__ void copy_tile(const KDesc& d, uint32_t tile) {
   const uint32_t tid = threadIdx.x;
@@ -224,7 +374,7 @@ __device__ __forceinline__ void copy_tile(const KDesc& d, uint32_t tile) {
     } else {
       const uint32_t nvec = tile_bytes / 16;
       for (uint32_t c = tid; c < nvec; c += kThreads) st16_out<kPack>(dst + (size_t)c * 16, ld16(src + (size_t)c * 16));
-      for (uint32_t b = nvec * 16 + tid * eb; b < tile_bytes; b += kThreads * eb) copy_elem<kG, kG>(dst + b, src + b, eb);
+      for (uint32_t b = nvec * 16 + tid * eb; b < tile_bytes; b += kThreads * eb) copy_elem(dst + b, src + b, eb);
     }
     return;
   }
@@ -257,9 +407,9 @@ __device__ __forceinline__ void copy_tile(const KDesc& d, uint32_t tile) {
       for (uint32_t c = tid; c < nvec; c += kThreads) narrow_chunk<kPack>(payload + (size_t)c * 16, t + (size_t)c * 32);
       for (uint32_t b = nvec * 16 + tid * 2; b < tile_bytes; b += kThreads * 2) {
         if (kPack)
-          st<kG>(payload + b, (uint16_t)(ld<kG, uint32_t>(t + (size_t)b * 2) >> 16));
+          st(payload + b, (uint16_t)(ld<uint32_t>(t + (size_t)b * 2) >> 16));
         else
-          st<kG>(t + (size_t)b * 2, (uint32_t)ld<kG, uint16_t>(payload + b) << 16);
+          st(t + (size_t)b * 2, (uint32_t)ld<uint16_t>(payload + b) << 16);
       }
     }
     return;
@@ -290,30 +440,16 @@ __device__ __forceinline__ void copy_tile(const KDesc& d, uint32_t tile) {
     return;
   }
 
-  if constexpr (kElem) copy_tile_elem<kPack>(d, tile_off, tile_bytes, payload, tensor, eb, tid);
-}
-
-// ELEM: LDS-staged element gather / scatter of one tile.
-template <bool kPack>
-__device__ __forceinline__ void copy_tile_elem(const KDesc& d, uint64_t tile_off, uint32_t tile_bytes, char* payload,
-                                               char* tensor, uint32_t eb, uint32_t tid) {
-  __shared__ uint4 lds[kTileBytes / 16];
-  char* const sbuf = (char*)lds;
-  const uint32_t nelem = tile_bytes / eb;
-  const uint32_t e0 = (uint32_t)d.first + (uint32_t)(tile_off / eb);
-  const uint32_t nvec = tile_bytes / 16;
-  if (kPack) {
-    for (uint32_t j = tid; j < nelem; j += kThreads)
-      copy_elem<kL, kG>(sbuf + (size_t)j * eb, tensor + unit_offset(d, e0 + j), eb);
-    __syncthreads();
-    for (uint32_t c = tid; c < nvec; c += kThreads) st16_stream(payload + (size_t)c * 16, ld<kL, uint4>(sbuf + (size_t)c * 16));
-    for (uint32_t b = nvec * 16 + tid * eb; b < tile_bytes; b += kThreads * eb) copy_elem<kG, kL>(payload + b, sbuf + b, eb);
-  } else {
-    for (uint32_t c = tid; c < nvec; c += kThreads) st<kL>(sbuf + (size_t)c * 16, ld16(payload + (size_t)c * 16));
-    for (uint32_t b = nvec * 16 + tid * eb; b < tile_bytes; b += kThreads * eb) copy_elem<kL, kG>(sbuf + b, payload + b, eb);
-    __syncthreads();
-    for (uint32_t j = tid; j < nelem; j += kThreads)
-      copy_elem<kG, kL>(tensor + unit_offset(d, e0 + j), sbuf + (size_t)j * eb, eb);
+  if constexpr (kElem) {
+    __shared__ uint4 lds[kTileBytes / 16];
+    const uint32_t e0 = (uint32_t)d.first + (uint32_t)(tile_off / eb);
+    if (d.path == kPathRows) {
+      rows_tile<kPack>(d, e0, tile_bytes, payload, tensor, eb, tid);
+    } else {
+      with_element(eb, [&](auto zero) {
+        elem_tile<kPack, decltype(zero)>(d, e0, tile_bytes, payload, tensor, tid, (MO_LDS char*)lds);
+      });
+    }
   }
 }
 
@@ -338,7 +474,7 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_unpack_kernel(cons
   mo::copy_body<false, false>(args);
 }
 
-// The same with ELEM pieces in the launch (16 KiB of LDS a workgroup).
+// The same with ROWS or ELEM pieces in the launch (16 KiB of LDS a workgroup).
 extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_pack_elem_kernel(const mo::LaunchArgs args) {
   mo::copy_body<true, true>(args);
 }
@@ -395,9 +531,9 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_equal_kernel(const
       diff |= (u.x ^ v.x) | (u.y ^ v.y) | (u.z ^ v.z) | (u.w ^ v.w);
     }
     for (uint32_t i = nvec * 16 + tid; i < (uint32_t)left; i += kThreads)
-      diff |= (uint32_t)(ld<kG, uint8_t>(x + i) ^ ld<kG, uint8_t>(y + i));
+      diff |= (uint32_t)(ld<uint8_t>(x + i) ^ ld<uint8_t>(y + i));
   }
-  if (diff) st<kG>((char*)flag, 1u);
+  if (diff) st((char*)flag, 1u);
 }
 
 // Device <-> pinned-host copy through the shader engines instead of a DMA engine.
@@ -419,7 +555,7 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_link_copy_kernel(c
   }
   for (; base < nvec; base += lanes) st16(dst + base * 16, ld16(src + base * 16));
   if (blockIdx.x == 0) {
-    for (uint64_t b = nvec * 16 + threadIdx.x; b < nbytes; b += kThreads) st<kG>(dst + b, ld<kG, uint8_t>(src + b));
+    for (uint64_t b = nvec * 16 + threadIdx.x; b < nbytes; b += kThreads) st(dst + b, ld<uint8_t>(src + b));
   }
 }
 
@@ -677,7 +813,7 @@ extern "C" __global__ __launch_bounds__(mo::kWireScanThreads) void mo_wire_scan_
   const uint64_t tail = raw_bytes % kWireBlockBytes, tail_src = wire_blocks(raw_bytes) * kWireBlockBytes;
   const uint64_t data_start = wire_data_start(raw_bytes);
   for (uint64_t i = tid; i < tail; i += kWireScanThreads)
-    __builtin_amdgcn_raw_buffer_store_b8(ld<kG, uint8_t>(raw + tail_src + i), w, (int)(data_start + i), 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b8(ld<uint8_t>(raw + tail_src + i), w, (int)(data_start + i), 0, 0);
   uint64_t carry = wire_tiles_start(raw_bytes);
   for (uint64_t base = 0; base < tiles; base += kChunk) {
     const uint64_t t = base + 4 * tid;
@@ -710,7 +846,7 @@ extern "C" __global__ __launch_bounds__(mo::kWireScanThreads) void mo_wire_scan_
     __builtin_amdgcn_raw_buffer_store_b32((uint32_t)(carry >> 32), w, 4, 0, 0);
     __builtin_amdgcn_raw_buffer_store_b32((uint32_t)raw_bytes, w, 8, 0, 0);
     __builtin_amdgcn_raw_buffer_store_b32((uint32_t)tiles, w, 12, 0, 0);
-    if (host_total) st<kG>((char*)host_total, carry);
+    if (host_total) st((char*)host_total, carry);
   }
 }
 
@@ -820,7 +956,7 @@ extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const cha
     const uint64_t tail = raw_bytes % kWireBlockBytes, tail_dst = wire_blocks(raw_bytes) * kWireBlockBytes;
     const uint64_t data_start = wire_data_start(raw_bytes);
     for (uint64_t i = lane; i < tail; i += 64)
-      st<kG>(raw + tail_dst + i, (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(w, (int)(data_start + i), 0, 0));
+      st(raw + tail_dst + i, (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(w, (int)(data_start + i), 0, 0));
   }
   const uint64_t tile = blockIdx.x;
   if (tile >= wire_tiles(raw_bytes)) return;

@@ -22,7 +22,7 @@ constexpr uint64_t kNoAllocScratchBytes = 64ull << 20;
 
 // NARROW: contiguous float32 on the tensor side, its high halves (bfloat16 bits) as the
 // payload; `first` and `nbytes` count payload bytes, the tensor side is twice that.
-enum : uint8_t { kPathContig = 0, kPathRuns = 1, kPathElem = 2, kPathNarrow = 3 };
+enum : uint8_t { kPathContig = 0, kPathRuns = 1, kPathElem = 2, kPathNarrow = 3, kPathRows = 4 };
 
 // Cache policy of a piece (KDesc::cache): non-temporal loads of the side read (the tensor when
 // packing, the payload when unpacking) and non-temporal stores of the side written. Streaming

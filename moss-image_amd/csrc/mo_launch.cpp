@@ -35,7 +35,7 @@ struct DeviceModule {
   hipModule_t module = nullptr;
   hipFunction_t pack = nullptr, unpack = nullptr, link = nullptr;
   hipFunction_t pack1 = nullptr, unpack1 = nullptr;  // single-piece launches
-  // the same four with ELEM pieces in the launch (they reserve the LDS staging buffer)
+  // the same four with ROWS or ELEM pieces in the launch (they reserve the LDS staging buffer)
   hipFunction_t pack_elem = nullptr, unpack_elem = nullptr, pack1_elem = nullptr, unpack1_elem = nullptr;
   hipFunction_t equal = nullptr;
   hipFunction_t wire_sizes = nullptr, wire_scan = nullptr, wire_encode = nullptr, wire_decode = nullptr;
@@ -176,13 +176,16 @@ int make_kdesc(const Canon& c, uint64_t tensor_base, uint64_t first, uint64_t nb
     }
     return 0;
   }
-  // ELEM path: units are elements; the innermost canonical dim is the inner run.
+  // ROWS (contiguous runs off the 16-byte grid) and ELEM (an element-strided innermost dim): units
+  // are elements; the innermost canonical dim is the inner run.
   if (c.numel >= (1ull << 32)) {
     err = "tensor too large for 32-bit element indexing";
     return MO_E_INVALID;
   }
   const int eouter = nd > 0 ? nd - 1 : 0;
-  kd.path = kPathElem;
+  // a chunk meets at most one run end while runs hold 16 bytes, and ROWS handles one; rows of three
+  // int64 (24 bytes) already measure alike on both
+  kd.path = inner_contig && nd > 0 && run_bytes >= 16 ? kPathRows : kPathElem;
   kd.first = first / c.eb;
   if (nd == 0) {
     kd.inner_stride = c.eb;
@@ -222,7 +225,7 @@ void Launcher::add(const KDesc& kd) {
   bytes_ += kd.nbytes;
   pending_bytes_ += kd.nbytes;
   pending_hbm_ += kd.nbytes * (kd.path == kPathNarrow ? 3 : 2);  // narrow: 2 B tensor-side per payload B
-  has_elem_ = has_elem_ || kd.path == kPathElem;
+  has_elem_ = has_elem_ || kd.path == kPathElem || kd.path == kPathRows;
   args_.ndesc++;
   if (tiles_ > kMaxTilesPerLaunch) flush();
 }

@@ -180,3 +180,42 @@ def test_bf16_high_gather_keeps_the_high_halves_and_scatter_restores_the_bits(nu
     _native.check("mo_scatter", lib.mo_scatter(back, 2, payload.data_ptr(), None, stream))
     assert_bitwise(out, t)
     assert_bitwise(out_plain, plain)
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32, torch.int64, torch.complex128])
+def test_runs_off_the_16_byte_grid(dtype) -> None:
+    """Contiguous runs that 16-byte chunks do not divide: run lengths at and around one chunk and
+    one tile's lane stride, pieces that end at every remainder of a chunk, rows of a tile and one
+    element more, and starts off the grid; in one launch, then each as a launch of one piece."""
+
+    device = torch.device("cuda", 0)
+    eb = torch.empty((), dtype=dtype).element_size()
+    per = 16 // eb  # elements of a chunk
+    views = []
+    for k, (rows, run, gap, offset) in enumerate([
+            (37, per, 1, 0), (37, per + 1, 1, 1), (5, 2 * per - 1, per + 1, 1), (301, max(per - 1, 1), 1, 0),
+            (9, 256 * per + 1, 3, 1), (3, 1024 * per, 1, 1), (3, 1024 * per + 1, 1, 0), (1, 1024 * per - 1, 0, 1),
+            (1, 4096 + per + 1, 0, 1), (211, 67, 10, 0)]):
+        backing = random_bytes_tensor((offset + rows * (run + gap) + 4) * eb + 64, device, 77 + k)
+        views.append(view_of(backing, dtype, offset, (rows, run), (run + gap, 1)))
+        if run > per:  # the same runs over two outer dimensions
+            half = view_of(backing, dtype, offset, (max(rows // 2, 1), 2 if rows > 1 else 1, run - 1),
+                           (2 * (run + gap), run + gap, 1))
+            views.append(half)
+    views = [_offload_view(v)[0] for v in views]
+    if eb == 16:  # the oracle has no 16-byte elements: the same bytes as pairs of 8-byte ones
+        lib, stream = _native.load(), torch.cuda.current_stream(device).cuda_stream
+        descs = _descs(views)
+        offsets, total = _layout(lib, descs, len(views))
+        payload = torch.full((total,), 0xC3, dtype=torch.uint8, device=device)
+        _native.check("mo_gather", lib.mo_gather(descs, len(views), payload.data_ptr(), None, stream))
+        back = [torch.zeros_like(v) for v in views]
+        _native.check("mo_scatter", lib.mo_scatter(_descs(back), len(views), payload.data_ptr(), None, stream))
+        for v, b, off in zip(views, back, offsets):
+            pairs = torch.view_as_real(v).contiguous().view(torch.int64)
+            assert torch.equal(payload[off : off + 16 * v.numel()].view(torch.int64), pairs.reshape(-1))
+            assert torch.equal(torch.view_as_real(b).contiguous().view(torch.int64), pairs)
+        return
+    _round_trip(views, device)
+    for v in views:
+        _round_trip([v], device)
