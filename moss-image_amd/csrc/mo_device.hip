@@ -927,26 +927,29 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_wire_encode_kernel
 }
 
 // Decode a coded stream of `raw_bytes` into `raw`. Grid: max(tiles, 1) workgroups of one wave, a tile
-// each; the first also copies the raw tail. 8 KiB of LDS: each slot's rank, the table entries by
-// rank, a ring of the stream's next 512 words, and one group's exponents: state l decodes the
-// tile's words 64 j + l, so the exponents of 8 rounds are 1 KiB of consecutive words, written out
-// as one 16-byte store a lane.
-// Bound by a round's chain of three LDS reads (slot, entry, stream word) and the vector instructions
-// between them, and with 13.5 waves a CU (113 MB) nearly as much by the issue of those: so a round
-// is kept short. A wave is its own workgroup (its arrays lie at fixed LDS addresses; 13.5 waves a
-// CU also spread better than 3.4 groups of four); an entry's parts sit where the multiply, the
-// subtraction and the byte store take them as they are; the ring repeats its first 256 words past
-// its end, so that the four rounds between refills index it without wrapping; and a byte select
-// brings a stream word in. 113 MB: 67 us with four
-// tiles a workgroup and 26 instructions a round, now 53.5; a 256 KiB segment 48, now 33.
+// each; the first also copies the raw tail. In LDS: the slots' table, the entries by rank (2 KiB), a
+// ring of the stream's next 512 words, and one group's exponents: state l decodes the tile's words
+// 64 j + l, so the exponents of 8 rounds are 1 KiB of consecutive words, written out as one 16-byte
+// store a lane.
+// Bound by a round's chain of LDS reads and the vector instructions between them, and where a CU
+// holds many tiles nearly as much by the issue of those: so a round is kept short. A wave is its own
+// workgroup (its arrays lie at fixed LDS addresses, and tiles spread evenly over the CUs); the ring
+// repeats its first 256 words past its end, so that the four rounds between refills index it without
+// wrapping; and a byte select brings a stream word in.
+// kDirect: the slots' table holds whole entries (16 KiB; 20 KiB a tile, 8 tiles a CU), two LDS reads
+// a round. Otherwise it holds ranks (4 KiB; 8 KiB a tile, 20 tiles a CU), whose entries a third read
+// brings; an entry's parts sit where the multiply, the subtraction and the byte store take them as
+// they are. 113 MB: 67 us with four tiles a workgroup and 26 instructions a round, 53.5 by ranks now;
+// a 256 KiB segment 48 us, 33 by ranks, 29.7 direct.
 // Reads go through a resource over [wire, wire + wire_bytes), and writes stay inside
 // [raw, raw + raw_bytes) whatever the stream holds: a damaged header is clamped, and table values
 // only index the wave's own LDS arrays.
-extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const char* wire, uint64_t wire_bytes,
-                                                                       uint64_t raw_bytes, char* raw) {
-  using namespace mo;
+namespace mo {
+template <bool kDirect>
+__device__ __forceinline__ void wire_decode_body(const char* wire, uint64_t wire_bytes, uint64_t raw_bytes, char* raw) {
   constexpr uint32_t kSlots = 1u << kWireProbBits, kRing = 512, kAgain = 256;
-  __shared__ __attribute__((aligned(16))) unsigned char slot_rank[kSlots];
+  // a slot's rank (a byte), or with kDirect its entry: slot - c | exponent << 12 | f - 1 << 20
+  __shared__ __attribute__((aligned(16))) unsigned char slots[kDirect ? 4 * kSlots : kSlots];
   __shared__ __attribute__((aligned(16))) mo_u32x2 rank_entry[256];  // {f, c | exponent << 16}
   __shared__ __attribute__((aligned(16))) unsigned short ring[kRing + kAgain];
   __shared__ __attribute__((aligned(16))) unsigned char group[8 * kWireLanes];
@@ -973,14 +976,14 @@ extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const cha
     return;
   }
   const uint32_t nsym = min((head >> 8) & 0x1ffu, 256u);
-  MO_LDS unsigned char* const sr = (MO_LDS unsigned char*)slot_rank;
+  MO_LDS unsigned char* const sr = (MO_LDS unsigned char*)slots;
   MO_LDS mo_u32x2* const re = (MO_LDS mo_u32x2*)rank_entry;
   MO_LDS unsigned short* const words = (MO_LDS unsigned short*)ring;
   MO_LDS unsigned char* const grp = (MO_LDS unsigned char*)group;
   // Table entries in rank order with their cumulative frequencies; each entry's first slot is
   // marked with its rank (rank 0 starts at slot 0, where every slot's mark starts).
   const uint32_t tab = body + n;
-  for (uint32_t i = lane; i < kSlots / 16; i += 64) *(MO_LDS mo_u32x4*)(sr + 16 * i) = mo_u32x4{0, 0, 0, 0};
+  for (uint32_t i = lane; i < sizeof(slots) / 16; i += 64) *(MO_LDS mo_u32x4*)(sr + 16 * i) = mo_u32x4{0, 0, 0, 0};
   wave_lds_fence();
   uint32_t carry = 0;
 #pragma unroll
@@ -991,23 +994,42 @@ extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const cha
     const uint32_t incl = wave_scan(f, lane), c = carry + incl - f;
     carry += (uint32_t)__shfl((int)incl, 63, 64);
     re[r] = mo_u32x2{f, (c & 0xffffu) | ((e & 0xffu) << 16)};
-    if (f && c < kSlots) sr[c] = (unsigned char)r;
+    if (f && c < kSlots) sr[kDirect ? 4 * c : c] = (unsigned char)r;
   }
   wave_lds_fence();
   // Every slot's rank: the last mark at or before it (marks rise with the slot). Four consecutive
-  // slots a lane: the byte maxima within its word, a prefix maximum over the lanes' last bytes, and
-  // the carry of the rounds before.
+  // slots a lane: the maxima within them, a prefix maximum over the lanes' last ones, and the carry
+  // of the rounds before.
   uint32_t before = 0;
   for (uint32_t row = 0; row < kSlots / 256; ++row) {
-    const uint32_t four = *(const MO_LDS uint32_t*)(sr + 256 * row + 4 * lane);
     uint32_t m[4];
-    m[0] = four & 0xffu;
+    if (kDirect) {
+      const mo_u32x4 four = *(const MO_LDS mo_u32x4*)(sr + 1024 * row + 16 * lane);
 #pragma unroll
-    for (int k = 1; k < 4; ++k) m[k] = max(m[k - 1], (four >> (8 * k)) & 0xffu);
+      for (int k = 0; k < 4; ++k) m[k] = four[k];
+    } else {
+      const uint32_t four = *(const MO_LDS uint32_t*)(sr + 256 * row + 4 * lane);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) m[k] = (four >> (8 * k)) & 0xffu;
+    }
+#pragma unroll
+    for (int k = 1; k < 4; ++k) m[k] = max(m[k - 1], m[k]);
     const uint32_t upto = wave_scan_max_dpp(m[3]);
     const uint32_t left = max(before, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)upto, 0x138, 0xf, 0xf, false));  // wave_shr:1
-    *(MO_LDS uint32_t*)(sr + 256 * row + 4 * lane) =
-        max(left, m[0]) | (max(left, m[1]) << 8) | (max(left, m[2]) << 16) | (max(left, m[3]) << 24);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) m[k] = max(left, m[k]);
+    if (kDirect) {
+      mo_u32x4 entries;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const mo_u32x2 t = re[m[k]];
+        const uint32_t f = t[0], ce = t[1];
+        entries[k] = ((256 * row + 4 * lane + k - ce) & 0xfffu) | ((ce >> 16) << 12) | ((f - 1) << 20);
+      }
+      *(MO_LDS mo_u32x4*)(sr + 1024 * row + 16 * lane) = entries;
+    } else {
+      *(MO_LDS uint32_t*)(sr + 256 * row + 4 * lane) = m[0] | (m[1] << 8) | (m[2] << 16) | (m[3] << 24);
+    }
     before = max(before, (uint32_t)__builtin_amdgcn_readlane((int)upto, 63));
   }
   // States, and the stream's first 512 words into the ring (word i at i % 512, and again at
@@ -1040,10 +1062,18 @@ extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const cha
     wrap();
 #pragma unroll
     for (uint32_t r = 0; r < 8; ++r) {
-      const uint32_t slot = x % kSlots;
-      const mo_u32x2 t = re[sr[slot]];
-      const uint32_t f = t[0], ce = t[1];
-      x = __umul24(f, x >> kWireProbBits) + (slot - (ce & 0xffffu));
+      const uint32_t slot = x % kSlots, high = x >> kWireProbBits;
+      uint32_t exponent;
+      if (kDirect) {
+        const uint32_t t = *(const MO_LDS uint32_t*)(sr + 4 * slot);
+        x = __umul24(t >> 20, high) + (high + (t & 0xfffu));
+        exponent = t >> 12;
+      } else {
+        const mo_u32x2 t = re[sr[slot]];
+        const uint32_t f = t[0], ce = t[1];
+        x = __umul24(f, high) + (slot - (ce & 0xffffu));
+        exponent = ce >> 16;
+      }
       const bool need = x < kWireStateLow;
       const uint64_t bal = __ballot(need);
       const uint32_t mine = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
@@ -1051,7 +1081,7 @@ extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const cha
       x = __builtin_amdgcn_perm(x, word, need ? 0x05040100u : 0x07060504u);  // (x << 16) | word, or x
       ptr += (uint32_t)__popcll(bal);
       at += 2 * (uint32_t)__popcll(bal);
-      grp[64 * r + lane] = (unsigned char)(ce >> 16);
+      grp[64 * r + lane] = (unsigned char)exponent;
       // Every four rounds, which read at most 256 words: the ring holds at least 512 - 127 of them.
       // Words [wb, wb + 128) are consumed: their ring quarter takes words [wb + 512, wb + 640).
       if (r % 4 == 3) {
@@ -1076,4 +1106,15 @@ extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const cha
     st16(dst + 1024 * (uint64_t)g + 16 * lane, make_uint4(o[0], o[1], o[2], o[3]));
     wave_lds_fence();  // the group buffer is read before the next group writes it
   }
+}
+}  // namespace mo
+
+extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_kernel(const char* wire, uint64_t wire_bytes,
+                                                                       uint64_t raw_bytes, char* raw) {
+  mo::wire_decode_body<false>(wire, wire_bytes, raw_bytes, raw);
+}
+
+extern "C" __global__ __launch_bounds__(64) void mo_wire_decode_direct_kernel(const char* wire, uint64_t wire_bytes,
+                                                                              uint64_t raw_bytes, char* raw) {
+  mo::wire_decode_body<true>(wire, wire_bytes, raw_bytes, raw);
 }

@@ -39,6 +39,8 @@ struct DeviceModule {
   hipFunction_t pack_elem = nullptr, unpack_elem = nullptr, pack1_elem = nullptr, unpack1_elem = nullptr;
   hipFunction_t equal = nullptr;
   hipFunction_t wire_sizes = nullptr, wire_scan = nullptr, wire_encode = nullptr, wire_decode = nullptr;
+  hipFunction_t wire_decode_direct = nullptr;
+  uint64_t direct_tiles = 0;  // segments of at most this many tiles are decoded by it
   // this device's copy of mo_noalloc_scratch (every device holds its own, at its own address)
   uint64_t scratch = 0, scratch_bytes = 0;
 };
@@ -63,6 +65,12 @@ int load_functions(DeviceModule& m) {
   if ((e = hipModuleGetFunction(&m.wire_scan, m.module, "mo_wire_scan_kernel")) != hipSuccess) return (int)e;
   if ((e = hipModuleGetFunction(&m.wire_encode, m.module, "mo_wire_encode_kernel")) != hipSuccess) return (int)e;
   if ((e = hipModuleGetFunction(&m.wire_decode, m.module, "mo_wire_decode_kernel")) != hipSuccess) return (int)e;
+  if ((e = hipModuleGetFunction(&m.wire_decode_direct, m.module, "mo_wire_decode_direct_kernel")) != hipSuccess)
+    return (int)e;
+  int device = 0, cus = 0;
+  if ((e = hipGetDevice(&device)) != hipSuccess) return (int)e;
+  if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device)) != hipSuccess) return (int)e;
+  m.direct_tiles = (uint64_t)cus * kWireDirectTilesPerCu;
   // Set-up of the allocation-free entry point, once per device with that device current: the
   // device address of this module's scratch array. From here on only this address is used.
   hipDeviceptr_t scratch = nullptr;
@@ -348,8 +356,12 @@ int wire_decode(uint64_t wire, uint64_t wire_bytes, uint64_t raw, uint64_t raw_b
   void* r = (void*)raw;
   uint64_t wb = wire_bytes, n = raw_bytes;
   void* params[] = {&w, &wb, &n, &r};
-  return (int)hipModuleLaunchKernel(m.wire_decode, tiles ? (uint32_t)tiles : 1, 1, 1, kWireLanes, 1, 1, 0, stream,
-                                    params, nullptr);  // a wave per tile
+  // Whole entries a slot while every tile is resident with them (8 a CU: 64 MiB on 256 CUs): 256 KiB
+  // 32.7 us by ranks and 29.7 direct, 16 MiB 37.1 and 34.6, 63 MiB 43.4 and 41.3. One tile more
+  // waits for a whole tile's time: 72 MiB 45.9 by ranks, 69.5 direct.
+  const hipFunction_t fn = tiles <= m.direct_tiles ? m.wire_decode_direct : m.wire_decode;
+  return (int)hipModuleLaunchKernel(fn, tiles ? (uint32_t)tiles : 1, 1, 1, kWireLanes, 1, 1, 0, stream, params,
+                                    nullptr);  // a wave per tile
 }
 
 }  // namespace mo

@@ -54,6 +54,7 @@ constexpr uint32_t kWireLanes = 64;           // interleaved rANS states per til
 constexpr uint32_t kWireProbBits = 12;        // frequencies sum to 4096
 constexpr uint32_t kWireStateLow = 1u << 16;  // states stay in [2^16, 2^32)
 constexpr uint32_t kWireModeRans = 0, kWireModeRaw = 1;
+constexpr uint32_t kWireDirectTilesPerCu = 8;  // decode: tiles whose whole-entry tables a CU's LDS holds
 constexpr uint32_t kWireTilesPerGroup = 4;   // coded sizes: one wave per tile, four waves a workgroup
 constexpr uint32_t kWireScanThreads = 1024;  // the one workgroup of the offset scan
 // Working space per tile: record, table (256 u32), states, stream (one word per exponent).

@@ -126,9 +126,11 @@ def test_large_gaussian_buffer_round_trip_and_ratio() -> None:
     assert torch.equal(out.view(torch.int16), src.view(torch.int16))
 
 
-@pytest.mark.parametrize("tiles,distinct", [(4097, 3), (4096, 40), (33, 256), (5, 1)])
+@pytest.mark.parametrize("tiles,distinct", [(4097, 3), (4096, 40), (33, 256), (5, 1), (2048, 25), (2049, 25),
+                                            (2049, 256), (2049, 1)])
 def test_tile_counts_and_alphabets_round_trip(tiles, distinct) -> None:
-    """Tile counts at the edge of the offset scan's chunk (4 096 tiles, 128 MiB) and past it, and
+    """Tile counts at the edge of the offset scan's chunk (4 096 tiles, 128 MiB) and past it, at the
+    edge of the decoder's whole-entry tables (8 tiles a CU of 256) and past it, and
     tables of 1, a few and all 256 exponents (the kernel's table, state and stream copies start at
     every 4-byte position of those sizes): the tile offsets rise by whole 16-byte pieces to the
     coded size, and the round trip is bitwise."""
