@@ -161,8 +161,10 @@ def decode_transposed_hip(weight: torch.Tensor, scale: torch.Tensor) -> torch.Te
     return out
 
 
-def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: int, backward: bool) -> str:
-    """The path a call takes: ``strip``, ``library``, ``transposed`` or ``fused``."""
+def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: int, backward: bool,
+           *operands: torch.Tensor | None) -> str:
+    """The path a call takes: ``strip``, ``library``, ``transposed`` or ``fused``. ``operands``: the
+    activation matrix and the output buffer (None: a new one)."""
 
     if path not in PATHS:
         raise ValueError(f"path must be one of {PATHS}")
@@ -171,13 +173,18 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
     if path != "auto":
         return path
     long_reduction = reduction >= LONG_REDUCTION * width
-    if reduction % 64 == 0 and _strips(rows, reduction, width, backward, long_reduction):
+    # What the strip kernels' and the transposed decode's argument checks refuse and the library path
+    # takes (activations or outputs off the 16-byte grid, no rows, larger weights) stays with it.
+    fits = weight.numel() < 1 << 31 and all(size % 16 == 0 and size <= 1 << 20 for size in weight.shape)
+    aligned = all(t is None or t.data_ptr() % 16 == 0 for t in operands)
+    if (rows and fits and aligned and reduction % 64 == 0
+            and _strips(rows, reduction, width, backward, long_reduction)):
         return "strip"
     if rows < LIBRARY_ROWS and weight.numel() < LIBRARY_WEIGHT:
         return "fused"
     if long_reduction and _splits(rows, width, reduction, backward):
         return "fused"
-    if backward and reduction >= TRANSPOSED_REDUCTION and not long_reduction and width & (width - 1):
+    if backward and fits and reduction >= TRANSPOSED_REDUCTION and not long_reduction and width & (width - 1):
         return "transposed"
     return "library"
 
@@ -236,7 +243,7 @@ def int8_linear_forward(tokens: torch.Tensor, weight: torch.Tensor, scale: torch
     out_features = weight.shape[0]
     if bias is not None:
         bias = bias.to(torch.bfloat16).contiguous()
-    route = _route(path, rows, weight, in_features, out_features, False)
+    route = _route(path, rows, weight, in_features, out_features, False, matrix, out)
     if route == "library":
         decoded = decode_hip(weight, scale)
         if out is None:
@@ -273,7 +280,7 @@ def int8_linear_backward(gradient: torch.Tensor, weight: torch.Tensor, scale: to
     matrix = gradient.reshape(-1, gradient.shape[-1]).to(torch.bfloat16).contiguous()
     rows, out_features = matrix.shape
     in_features = weight.shape[1]
-    route = _route(path, rows, weight, out_features, in_features, True)
+    route = _route(path, rows, weight, out_features, in_features, True, matrix, out)
     if route == "transposed":
         decoded = decode_transposed_hip(weight, scale)
         if out is None:

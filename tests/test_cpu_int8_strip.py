@@ -6,6 +6,7 @@ from __future__ import annotations
 import random
 
 import pytest
+import torch
 
 from moss_offload import _native, quant_kernels as qk
 
@@ -51,3 +52,27 @@ def test_every_plan_keeps_its_invariants() -> None:
         assert alone["splits"] == 1 and alone["split_steps"] == steps
     with pytest.raises(_native.EngineError):
         qk.strip_plan(64, 64, 80, CUS)
+
+
+@pytest.mark.parametrize("backward", [False, True])
+def test_route_leaves_the_library_what_the_strips_refuse(backward) -> None:
+    """Weights of the library path's size: calls that the kernels' argument checks refuse."""
+
+    weight = torch.empty(6144, 3072, dtype=torch.int8, device="meta")
+    reduction, width = (6144, 3072) if backward else (3072, 6144)
+    flat = torch.empty(320 * reduction + 8, dtype=torch.bfloat16)
+    grid, off = flat[: 320 * reduction], flat[1 : 1 + 320 * reduction]
+    assert grid.data_ptr() % 16 == 0
+    take = ("library", "transposed") if backward else ("library",)
+
+    def route(rows, weight, *operands):
+        return qk._route("auto", rows, weight, reduction, width, backward, *operands)
+
+    assert route(320, weight, grid, None) == route(320, weight, grid, grid) == "strip"
+    assert route(320, weight, off, None) in take and route(320, weight, grid, off) in take
+    assert route(0, weight, grid[:0], None) in take
+    odd = torch.empty(6152, 3072, dtype=torch.int8, device="meta")
+    huge = torch.empty(1 << 20, 2048, dtype=torch.int8, device="meta")
+    assert route(320, odd, grid, None) == route(320, huge, grid, None) == "library"
+    # calls of the fused kernels' size stay with them, and are refused there as before
+    assert route(320, weight[:3072], off, None) == "fused"
