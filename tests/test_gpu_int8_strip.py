@@ -115,3 +115,22 @@ def test_strip_refuses_what_it_cannot_run() -> None:
         x.data_ptr(), w.data_ptr(), scale.data_ptr(), 0, y.data_ptr(), 33, 3072, 1040, 0, 0, stream))
     decoded = quant_kernels.decode(w, scale, torch.bfloat16).double().t()
     _within_accumulation_bound(y, x.double() @ decoded, x.double().abs() @ decoded.abs(), 3072)
+
+
+def test_operands_off_the_grid_run_as_on_the_library_path() -> None:
+    rows, out_f, in_f = 33, 6144, 3072
+    x, w, scale, b = _operands(rows, in_f, out_f, seed=12, bias=True)
+    dy = _operands(rows, out_f, 16, seed=13)[0]
+    for backward, a, width in ((False, x, out_f), (True, dy, in_f)):
+        off = torch.empty(a.numel() + 1, dtype=torch.bfloat16, device=DEV)[1:].view(a.shape)
+        off.copy_(a)
+        out = torch.empty(rows * width + 1, dtype=torch.bfloat16, device=DEV)[1:]
+        decoded = quant_kernels.decode(w, scale, torch.bfloat16).double()
+        decoded = decoded if backward else decoded.t()
+        for matrix, buffer in ((off, None), (a, out)):
+            if backward:
+                got = quant_kernels.int8_linear_backward(matrix, w, scale, torch.Size((rows, width)), out=buffer)
+            else:
+                got = quant_kernels.int8_linear_forward(matrix, w, scale, b, out=buffer)
+            exact = a.double() @ decoded + (0 if backward else b.double())
+            _within_accumulation_bound(got, exact, a.double().abs() @ decoded.abs(), a.shape[1])
