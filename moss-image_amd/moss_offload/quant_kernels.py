@@ -143,6 +143,7 @@ def decode_hip(weight: torch.Tensor, scale: torch.Tensor, *, out: torch.Tensor |
     """``decode(weight, scale, bfloat16)`` in one HIP pass (``mo_int8_decode``), bit for bit."""
 
     lib = _native.load()
+    _check_weight(weight, scale)
     out_features, in_features = weight.shape
     out = _output(out, (out_features, in_features), weight.device, "decoded-weight")
     _native.check("mo_int8_decode", lib.mo_int8_decode(weight.data_ptr(), scale.data_ptr(), out.data_ptr(),
@@ -154,6 +155,7 @@ def decode_transposed_hip(weight: torch.Tensor, scale: torch.Tensor) -> torch.Te
     """``decode(weight, scale, bfloat16).t()``, contiguous, in one HIP pass, bit for bit."""
 
     lib = _native.load()
+    _check_weight(weight, scale)
     out_features, in_features = weight.shape
     out = torch.empty((in_features, out_features), dtype=torch.bfloat16, device=weight.device)
     _native.check("mo_int8_decode_transposed", lib.mo_int8_decode_transposed(
@@ -161,17 +163,45 @@ def decode_transposed_hip(weight: torch.Tensor, scale: torch.Tensor) -> torch.Te
     return out
 
 
+def _check_weight(weight: torch.Tensor, scale: torch.Tensor) -> None:
+    """Every path hands the weight and its scales to a kernel by address: what they must be for that."""
+
+    if weight.ndim != 2 or weight.dtype != torch.int8 or not weight.is_contiguous():
+        raise RuntimeError("HIP int8 weight must be a contiguous int8 matrix.")
+    if scale.dtype != torch.float32 or scale.numel() != weight.shape[0] or not scale.is_contiguous() \
+            or scale.device != weight.device:
+        raise RuntimeError("HIP int8 scale must be contiguous float32 on the weight's device, one a row of the weight.")
+
+
+def _misfit(matrix: torch.Tensor, weight: torch.Tensor, features: int, bias: torch.Tensor | None = None,
+            outputs: int = 0) -> str | None:
+    """Why the kernels that take the activations by address cannot read them (None when they can):
+    they rely on the sizes they are given."""
+
+    if matrix.dtype != torch.bfloat16 or matrix.device != weight.device or matrix.shape[1] != features:
+        return f"expected bfloat16 rows of {features} on the weight's device"
+    if bias is not None and (bias.numel() != outputs or bias.shape[-1:] != (outputs,) or bias.device != weight.device):
+        return f"expected a bias of {outputs} on the weight's device"
+    return None
+
+
 def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: int, backward: bool,
-           *operands: torch.Tensor | None) -> str:
+           *operands: torch.Tensor | None, misfit: str | None = None) -> str:
     """The path a call takes: ``strip``, ``library``, ``transposed`` or ``fused``. ``operands``: the
-    activation matrix and the output buffer (None: a new one)."""
+    activation matrix and the output buffer (None: a new one). ``misfit``: ``_misfit``'s reason; such
+    a call is left to torch's matrix product, which refuses it or, for a bias that broadcasts or a
+    matrix that autocast converts, takes it."""
 
     if path not in PATHS:
         raise ValueError(f"path must be one of {PATHS}")
     if path == "transposed" and not backward:
         raise ValueError("the transposed path is the input gradient's")
+    if misfit and path in ("strip", "fused"):
+        raise RuntimeError(f"HIP int8 operands do not fit: {misfit}.")
     if path != "auto":
         return path
+    if misfit:
+        return "library"
     long_reduction = reduction >= LONG_REDUCTION * width
     # What the strip kernels' and the transposed decode's argument checks refuse and the library path
     # takes (activations or outputs off the 16-byte grid, no rows, larger weights) stays with it.
@@ -238,12 +268,14 @@ def int8_linear_forward(tokens: torch.Tensor, weight: torch.Tensor, scale: torch
     ``LIBRARY_ROWS``)."""
 
     lib = _native.load()
+    _check_weight(weight, scale)
     matrix = tokens.reshape(-1, tokens.shape[-1]).contiguous()
-    rows, in_features = matrix.shape
-    out_features = weight.shape[0]
+    rows = matrix.shape[0]
+    out_features, in_features = weight.shape
     if bias is not None:
         bias = bias.to(torch.bfloat16).contiguous()
-    route = _route(path, rows, weight, in_features, out_features, False, matrix, out)
+    misfit = _misfit(matrix, weight, in_features, bias, out_features)
+    route = _route(path, rows, weight, in_features, out_features, False, matrix, out, misfit=misfit)
     if route == "library":
         decoded = decode_hip(weight, scale)
         if out is None:
@@ -277,10 +309,12 @@ def int8_linear_backward(gradient: torch.Tensor, weight: torch.Tensor, scale: to
     library GEMM on ``decode_transposed_hip``'s weight)."""
 
     lib = _native.load()
+    _check_weight(weight, scale)
     matrix = gradient.reshape(-1, gradient.shape[-1]).to(torch.bfloat16).contiguous()
-    rows, out_features = matrix.shape
-    in_features = weight.shape[1]
-    route = _route(path, rows, weight, out_features, in_features, True, matrix, out)
+    rows = matrix.shape[0]
+    out_features, in_features = weight.shape
+    route = _route(path, rows, weight, out_features, in_features, True, matrix, out,
+                   misfit=_misfit(matrix, weight, out_features))
     if route == "transposed":
         decoded = decode_transposed_hip(weight, scale)
         if out is None:

@@ -1,0 +1,106 @@
+"""What ``int8_linear_forward`` and ``int8_linear_backward`` do before a kernel is given addresses.
+
+The native library is replaced by one that notes the calls it gets, and the decodes by the eager
+one, so that routing, refusals and the torch products of the library paths run on the CPU.
+"""
+
+from __future__ import annotations
+
+import types
+
+import pytest
+import torch
+
+from moss_offload import quant_kernels as qk
+
+SIZES = {"small": (64, 128), "library": (16384, 1024)}  # out_features, in_features: below and above LIBRARY_WEIGHT
+
+
+class _Library:
+    """Notes the names of the calls; its workspace sizes are zero."""
+
+    def __init__(self) -> None:
+        self.names: list[str] = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            if "bytes" not in name:
+                self.names.append(name)
+            return 0
+
+        return call
+
+
+@pytest.fixture
+def library(monkeypatch) -> _Library:
+    lib = _Library()
+    monkeypatch.setattr(qk, "_native", types.SimpleNamespace(load=lambda: lib, check=lambda name, rc: None))
+    monkeypatch.setattr(qk, "_stream", lambda tensor: 0)
+
+    def eager(weight, scale, out=None):
+        return qk.decode(weight, scale, torch.bfloat16)
+
+    monkeypatch.setattr(qk, "decode_hip", eager)
+    monkeypatch.setattr(qk, "decode_transposed_hip", lambda weight, scale: eager(weight, scale).t().contiguous())
+    return lib
+
+
+def _operands(size: str, rows: int = 20):
+    out_features, in_features = SIZES[size]
+    g = torch.Generator().manual_seed(out_features + rows)
+    weight = torch.randint(-127, 128, (out_features, in_features), dtype=torch.int8, generator=g)
+    scale = 0.001 + 0.01 * torch.rand(out_features, generator=g)
+    return (torch.randn(rows, in_features, generator=g).bfloat16(), torch.randn(rows, out_features, generator=g).bfloat16(),
+            weight, scale)
+
+
+@pytest.mark.parametrize("size", SIZES)
+def test_calls_that_fit_reach_a_kernel_by_address(library, size) -> None:
+    x, dy, w, s = _operands(size)
+    qk.int8_linear_forward(x, w, s, torch.zeros(w.shape[0]))
+    qk.int8_linear_forward(x, w, s[:, None], torch.zeros(1, w.shape[0]))
+    qk.int8_linear_backward(dy, w, s, x.shape)
+    assert library.names == ["mo_int8_strip_forward", "mo_int8_strip_forward", "mo_int8_strip_backward"]
+
+
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("path", ["auto", "strip", "fused"])
+@pytest.mark.parametrize("fault", ["float32", "wide", "bias", "scale", "scale dtype", "weight", "gradient"])
+def test_operands_that_do_not_fit_raise_before_any_kernel(library, size, path, fault) -> None:
+    x, dy, w, s = _operands(size)
+    bias = None
+    if fault == "float32":
+        x = x.float()
+    elif fault == "wide":
+        x = torch.cat([x, x], 1)
+    elif fault == "bias":
+        bias = torch.zeros(16)
+    elif fault == "scale":
+        s = s[:16].clone()
+    elif fault == "scale dtype":
+        s = s.bfloat16()
+    elif fault == "weight":
+        w = w.t().contiguous().t()
+    with pytest.raises(RuntimeError):
+        if fault == "gradient":
+            qk.int8_linear_backward(dy[:, 16:], w, s, x.shape, path=path)
+        else:
+            qk.int8_linear_forward(x, w, s, bias, path=path)
+    assert library.names == []
+
+
+@pytest.mark.parametrize("shape", [(), (1,), (20, 16384)])
+def test_a_bias_that_broadcasts_is_added_by_torch(library, shape) -> None:
+    x, _, w, s = _operands("library")
+    bias = torch.randn(shape).bfloat16()
+    got = qk.int8_linear_forward(x, w, s, bias)
+    assert library.names == []
+    want = torch.nn.functional.linear(x, qk.decode(w, s, torch.bfloat16), bias)
+    assert torch.equal(got, want)
+
+
+def test_the_reference_interface_refuses_activations_of_another_type(library) -> None:
+    x, _, w, s = _operands("library")
+    with pytest.raises(RuntimeError):
+        qk.triton_int8_linear_forward(x.float(), w, s, None, torch.bfloat16, torch.bfloat16)
+    assert library.names == []
