@@ -154,12 +154,13 @@ constexpr uint32_t kLoopSteps = 6;       // the register kernel's loop runs step
 // The launch for rows [row0, row0 + n) that do not fill a round of large tiles: a split
 // reduction on the large tile when `steps` (the reduction in steps of 64; 0 = no split) allows
 // at least two splits of kMinSplitSteps, the tiles times the splits fit one round, and the
-// rows fill at least three quarters of their large tiles; the small tile otherwise. A split's
+// rows fill at least three quarters of their large tiles; the small tile otherwise, and for an
+// empty output (the workspace functions plan calls that the launches refuse). A split's
 // length is rounded up to whole loop iterations (the last split takes what remains), which
 // keeps the time of the longest split and launches fewer workgroups.
 Part short_part(uint32_t row0, uint32_t n, uint32_t cols, uint32_t steps, int cus) {
   const uint64_t tm = (n + kLarge - 1) / kLarge, tiles = tm * ((cols + kLarge - 1) / kLarge);
-  if (steps && 4ull * n >= 3ull * tm * kLarge && tiles <= (uint64_t)cus / 2) {
+  if (steps && tiles && 4ull * n >= 3ull * tm * kLarge && tiles <= (uint64_t)cus / 2) {
     uint64_t s = (uint64_t)cus / tiles;
     if (s > steps / kMinSplitSteps) s = steps / kMinSplitSteps;
     if (s >= 2) {

@@ -204,7 +204,8 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
         return "library"
     long_reduction = reduction >= LONG_REDUCTION * width
     # What the strip kernels' and the transposed decode's argument checks refuse and the library path
-    # takes (activations or outputs off the 16-byte grid, no rows, larger weights) stays with it.
+    # takes (activations or outputs off the 16-byte grid, no rows, larger weights) stays with it. No
+    # rows of a smaller weight stay with the fused kernels, which refuse them.
     fits = weight.numel() < 1 << 31 and all(size % 16 == 0 and size <= 1 << 20 for size in weight.shape)
     aligned = all(t is None or t.data_ptr() % 16 == 0 for t in operands)
     if (rows and fits and aligned and reduction % 64 == 0
@@ -212,6 +213,8 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
         return "strip"
     if rows < LIBRARY_ROWS and weight.numel() < LIBRARY_WEIGHT:
         return "fused"
+    if rows == 0:
+        return "library"
     if long_reduction and _splits(rows, width, reduction, backward):
         return "fused"
     if backward and fits and reduction >= TRANSPOSED_REDUCTION and not long_reduction and width & (width - 1):

@@ -104,3 +104,18 @@ def test_the_reference_interface_refuses_activations_of_another_type(library) ->
     with pytest.raises(RuntimeError):
         qk.triton_int8_linear_forward(x.float(), w, s, None, torch.bfloat16, torch.bfloat16)
     assert library.names == []
+
+
+@pytest.mark.parametrize("size", ["library", "long"])
+@pytest.mark.parametrize("backward", [False, True])
+def test_a_call_without_rows_asks_no_launch_plan(library, monkeypatch, size, backward) -> None:
+    monkeypatch.setattr(qk, "_splits", lambda *args: pytest.fail("a plan of no tiles"))
+    shape = (16384, 1024)
+    if size == "long":  # the reduction at least four times the output width, in the call's direction
+        shape = (16384, 1024) if backward else (1024, 16384)
+    w, s = torch.zeros(shape, dtype=torch.int8), torch.ones(shape[0])
+    if backward:
+        got = qk.int8_linear_backward(torch.zeros(0, shape[0]).bfloat16(), w, s, torch.Size((0, shape[1])))
+    else:
+        got = qk.int8_linear_forward(torch.zeros(0, shape[1]).bfloat16(), w, s)
+    assert got.shape == (0, shape[1] if backward else shape[0]) and library.names == []

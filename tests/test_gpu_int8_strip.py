@@ -134,3 +134,23 @@ def test_operands_off_the_grid_run_as_on_the_library_path() -> None:
                 got = quant_kernels.int8_linear_forward(matrix, w, scale, b, out=buffer)
             exact = a.double() @ decoded + (0 if backward else b.double())
             _within_accumulation_bound(got, exact, a.double().abs() @ decoded.abs(), a.shape[1])
+
+
+@pytest.mark.parametrize("out_f,in_f", [(3072, 12288), (24576, 3072), (1024, 4096), (6144, 3072)])
+def test_calls_without_rows(out_f, in_f) -> None:
+    """Long and short reductions of either direction: the sizes are planned, small weights are refused."""
+
+    lib = _native.load()
+    assert lib.mo_int8_forward_workspace_bytes(0, in_f, out_f) == 0
+    assert lib.mo_int8_backward_workspace_bytes(0, in_f, out_f) == out_f * in_f  # the transposed weight
+    _, w, scale, _ = _operands(1, in_f, out_f, seed=14)
+    x = torch.empty(0, in_f, dtype=torch.bfloat16, device=DEV)
+    dy = torch.empty(0, out_f, dtype=torch.bfloat16, device=DEV)
+    if w.numel() < quant_kernels.LIBRARY_WEIGHT:
+        with pytest.raises(_native.EngineError):
+            quant_kernels.int8_linear_forward(x, w, scale)
+        with pytest.raises(_native.EngineError):
+            quant_kernels.int8_linear_backward(dy, w, scale, x.shape)
+    else:
+        assert quant_kernels.int8_linear_forward(x, w, scale).shape == (0, out_f)
+        assert quant_kernels.int8_linear_backward(dy, w, scale, x.shape).shape == (0, in_f)
