@@ -29,6 +29,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _native
 
@@ -185,12 +186,33 @@ def _misfit(matrix: torch.Tensor, weight: torch.Tensor, features: int, bias: tor
     return None
 
 
+def _by_address(*operands: torch.Tensor | None) -> bool:
+    """Whether a kernel that is given the operands' addresses does all that torch's product does with
+    them: there is no graph or tangent to carry on, and nothing that traces, batches or watches the
+    operators of the call."""
+
+    if torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() \
+            or torch._C._get_tracing_state() is not None:
+        return False
+    graph, dual = torch.is_grad_enabled(), forward_ad._current_level >= 0
+    for t in operands:
+        if t is None:
+            continue
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter or graph and t.requires_grad:
+            return False
+        if dual and forward_ad.unpack_dual(t).tangent is not None:
+            return False
+    return True
+
+
 def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: int, backward: bool,
-           *operands: torch.Tensor | None, misfit: str | None = None) -> str:
-    """The path a call takes: ``strip``, ``library``, ``transposed`` or ``fused``. ``operands``: the
-    activation matrix and the output buffer (None: a new one). ``misfit``: ``_misfit``'s reason; such
+           matrix: torch.Tensor, out: torch.Tensor | None, bias: torch.Tensor | None = None, *,
+           misfit: str | None = None) -> str:
+    """The path a call takes: ``strip``, ``library``, ``transposed`` or ``fused``. ``matrix``: the
+    activations; ``out``: the output buffer (None: a new one). ``misfit``: ``_misfit``'s reason; such
     a call is left to torch's matrix product, which refuses it or, for a bias that broadcasts or a
-    matrix that autocast converts, takes it."""
+    matrix that autocast converts, takes it. So is a call that is more than its bytes (see
+    ``_by_address``), unless it names a buffer, which no graph can go through."""
 
     if path not in PATHS:
         raise ValueError(f"path must be one of {PATHS}")
@@ -200,15 +222,19 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
         raise RuntimeError(f"HIP int8 operands do not fit: {misfit}.")
     if path != "auto":
         return path
-    if misfit:
+    plain = not misfit and _by_address(matrix, out, bias)
+    if misfit or not plain and out is None:
         return "library"
+    kind = matrix.device.type
+    if torch.is_autocast_enabled(kind) and torch.get_autocast_dtype(kind) != torch.bfloat16:
+        plain = False  # torch's product returns autocast's type, the strips bfloat16
     long_reduction = reduction >= LONG_REDUCTION * width
     # What the strip kernels' and the transposed decode's argument checks refuse and the library path
     # takes (activations or outputs off the 16-byte grid, no rows, larger weights) stays with it. No
     # rows of a smaller weight stay with the fused kernels, which refuse them.
     fits = weight.numel() < 1 << 31 and all(size % 16 == 0 and size <= 1 << 20 for size in weight.shape)
-    aligned = all(t is None or t.data_ptr() % 16 == 0 for t in operands)
-    if (rows and fits and aligned and reduction % 64 == 0
+    if (plain and rows and fits and reduction % 64 == 0 and matrix.data_ptr() % 16 == 0
+            and (out is None or out.data_ptr() % 16 == 0)
             and _strips(rows, reduction, width, backward, long_reduction)):
         return "strip"
     if rows < LIBRARY_ROWS and weight.numel() < LIBRARY_WEIGHT:
@@ -268,7 +294,8 @@ def int8_linear_forward(tokens: torch.Tensor, weight: torch.Tensor, scale: torch
     MFMA kernels for few rows; ``in_features`` a multiple of 64), ``fused`` (the MFMA kernels on
     large tiles), ``library`` (``decode_hip``, then the same ``addmm``/``mm`` as the reference's
     eager path, bit for bit), ``auto`` (by rows and shape, see ``STRIP_ROWS`` and
-    ``LIBRARY_ROWS``)."""
+    ``LIBRARY_ROWS``). The result of ``strip`` and ``fused`` has no graph; ``auto`` takes the library
+    path where one is wanted."""
 
     lib = _native.load()
     _check_weight(weight, scale)
@@ -278,7 +305,7 @@ def int8_linear_forward(tokens: torch.Tensor, weight: torch.Tensor, scale: torch
     if bias is not None:
         bias = bias.to(torch.bfloat16).contiguous()
     misfit = _misfit(matrix, weight, in_features, bias, out_features)
-    route = _route(path, rows, weight, in_features, out_features, False, matrix, out, misfit=misfit)
+    route = _route(path, rows, weight, in_features, out_features, False, matrix, out, bias, misfit=misfit)
     if route == "library":
         decoded = decode_hip(weight, scale)
         if out is None:

@@ -119,3 +119,85 @@ def test_a_call_without_rows_asks_no_launch_plan(library, monkeypatch, size, bac
     else:
         got = qk.int8_linear_forward(torch.zeros(0, shape[1]).bfloat16(), w, s)
     assert got.shape == (0, shape[1] if backward else shape[0]) and library.names == []
+
+
+def _call(backward, x, dy, w, s):
+    if backward:
+        return lambda t: qk.int8_linear_backward(t, w, s, t.shape[:-1] + (w.shape[1],)), dy
+    return lambda t: qk.int8_linear_forward(t, w, s), x
+
+
+@pytest.mark.parametrize("size,rows", [("library", 20), ("small", 20), ("small", 2100), ("small", 2700)])
+@pytest.mark.parametrize("backward", [False, True])
+def test_graphs_tangents_and_batches_go_through_the_product(library, size, backward, rows) -> None:
+    """Reverse mode, forward mode and vmap give what the product of the decoded weight gives, at
+    weights and rows of the strips' and of the library path."""
+
+    x, dy, w, s = _operands(size, rows)
+    call, t = _call(backward, x, dy, w, s)
+    decoded = qk.decode(w, s, torch.bfloat16)
+    linear = (lambda v: v @ decoded) if backward else (lambda v: v @ decoded.t())
+    leaf, tangent = t.clone().requires_grad_(True), torch.ones_like(t)
+
+    out = call(leaf)
+    (got,) = torch.autograd.grad(out.float().sum(), leaf)
+    other = t.clone().requires_grad_(True)
+    (want,) = torch.autograd.grad(linear(other).float().sum(), other)
+    assert torch.equal(got, want)
+    with torch.autograd.forward_ad.dual_level():
+        y = torch.autograd.forward_ad.unpack_dual(call(torch.autograd.forward_ad.make_dual(t, tangent))).tangent
+    assert torch.equal(y, linear(tangent))
+    assert torch.equal(torch.func.jvp(call, (t,), (tangent,))[1], linear(tangent))
+    assert torch.equal(torch.func.grad(lambda v: call(v).float().sum())(t), want)
+    assert torch.vmap(call)(torch.stack([t, tangent])).shape == (2, *linear(t).shape)
+    assert library.names == []
+    with torch.no_grad():  # nothing to carry on
+        assert not call(leaf).requires_grad
+    if rows == 20:
+        assert len(library.names) == 1
+
+
+def test_second_derivatives_go_through_the_frozen_linear(library, monkeypatch) -> None:
+    from moss_offload import dit
+
+    monkeypatch.setattr(qk, "unsupported_reason", lambda *args: None)
+    x, _, w, s = _operands("library")
+    module = dit.FrozenInt8Linear(w, s, torch.bfloat16, backend="hip")
+    first = module(x)
+    assert library.names == ["mo_int8_strip_forward"]
+    t, seed = x.clone().requires_grad_(True), torch.ones_like(first).requires_grad_(True)
+    (grad,) = torch.autograd.grad(module(t), t, seed, create_graph=True)
+    (second,) = torch.autograd.grad(grad.float().sum(), seed)
+    decoded = qk.decode(w, s, torch.bfloat16)
+    assert torch.equal(second, torch.ones_like(x) @ decoded.t())
+
+
+@pytest.mark.filterwarnings("ignore")  # torch.jit.trace is deprecated
+def test_what_watches_the_operators_sees_the_product(library) -> None:
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+
+    class Subclass(torch.Tensor):
+        pass
+
+    x, dy, w, s = _operands("library")
+    for backward in (False, True):
+        call, t = _call(backward, x, dy, w, s)
+        with FlopCounterMode(display=False) as counter:
+            call(t)
+        assert counter.get_total_flops() == 2 * 20 * w.numel()
+        assert "mm" in make_fx(call)(t).code
+        assert ("aten::matmul" if backward else "aten::linear") in str(torch.jit.trace(call, t, check_trace=False).graph)
+        assert type(call(t.as_subclass(Subclass))) is Subclass
+    assert library.names == []
+
+
+def test_autocast_to_another_type_keeps_its_result_type(library) -> None:
+    x, dy, w, s = _operands("library")
+    with torch.autocast("cpu", dtype=torch.float16):
+        assert qk.int8_linear_forward(x, w, s).dtype == torch.float16
+        assert qk.int8_linear_backward(dy, w, s, x.shape).dtype == torch.float16
+    assert library.names == []
+    with torch.autocast("cpu", dtype=torch.bfloat16):
+        assert qk.int8_linear_forward(x, w, s).dtype == torch.bfloat16
+    assert library.names == ["mo_int8_strip_forward"]
