@@ -799,13 +799,15 @@ __device__ __forceinline__ void strip_body(__bf16* a0, __bf16* a1, unsigned char
       }
     }
   }
-  float sf[CT];  // forward: bf16-rounded column scales
+  // forward: bf16-rounded column scales; zero from the end of the reduction on, where an infinite
+  // scale times the zero weights would be NaN
+  float sf[CT];
   if (!kBwd) {
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
       const int n = c0 + 32 * (CT * wn + ct) + lr;
       sf[ct] = bf16_round(__builtin_bit_cast(
-          float, __builtin_amdgcn_raw_buffer_load_b32(rs_src, n < N ? n * 4 : (int)kOob, 0, 0)));
+          float, __builtin_amdgcn_raw_buffer_load_b32(rs_src, any && n < N ? n * 4 : (int)kOob, 0, 0)));
     }
   }
 
@@ -913,6 +915,10 @@ __device__ __forceinline__ void strip_body(__bf16* a0, __bf16* a1, unsigned char
         if (kBwd) {  // step r0 + 128's scales, loaded a step ago; then the next load
           sbuf(b)[lane] = bf16_round(s_next);
           s_next = load_scale(r0 + 3 * kBR);
+        }
+        if (!kBwd) {
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) sf[ct] = r0 + kBR < klen ? sf[ct] : 0.f;
         }
         dma(abuf(b), wbuf(b), r0 + 2 * kBR);
       }

@@ -154,3 +154,45 @@ def test_calls_without_rows(out_f, in_f) -> None:
     else:
         assert quant_kernels.int8_linear_forward(x, w, scale).shape == (0, out_f)
         assert quant_kernels.int8_linear_backward(dy, w, scale, x.shape).shape == (0, in_f)
+
+
+@pytest.mark.parametrize("rows,cols,reduction", [c[:3] for c in CASES])
+@pytest.mark.parametrize("direction", ["forward", "backward"])
+def test_infinities_and_nans_stay_where_they_belong(rows, cols, reduction, direction) -> None:
+    """Positive operands, so that an infinite factor gives infinities and no NaN: the zeros that the
+    kernels multiply past a tile's edges, a K group's end and the last step must not meet it."""
+
+    g = torch.Generator().manual_seed(rows + cols)
+    x = (0.5 + torch.rand(rows, reduction, generator=g)).bfloat16().to(DEV)
+    shape = (cols, reduction) if direction == "forward" else (reduction, cols)
+    w = torch.randint(1, 128, shape, dtype=torch.int8, generator=g).to(DEV)
+    scale = (0.001 + 0.01 * torch.rand(shape[0], generator=g)).to(DEV)
+
+    def call(x, scale):
+        if direction == "forward":
+            return quant_kernels.int8_linear_forward(x, w, scale, path="strip")
+        return quant_kernels.int8_linear_backward(x, w, scale, torch.Size((rows, cols)), path="strip")
+
+    clean = call(x, scale)
+    assert clean.isfinite().all()
+    inf_row, nan_row = rows - 1, rows // 2
+    special = x.clone()
+    special[nan_row, reduction - 1] = float("nan")
+    special[inf_row, 0] = float("inf")  # the only row of a call of one: the infinity
+    if inf_row == nan_row:
+        special[inf_row, reduction - 1] = 1.0
+    got = call(special, scale)
+    assert (got[inf_row] == float("inf")).all()
+    assert inf_row == nan_row or got[nan_row].isnan().all()
+    other = torch.ones(rows, dtype=torch.bool, device=DEV)
+    other[[inf_row, nan_row]] = False
+    assert torch.equal(got[other].view(torch.int16), clean[other].view(torch.int16))
+
+    infinite = scale.clone()
+    infinite[-1] = float("inf")
+    got = call(x, infinite)
+    if direction == "forward":  # one column; the others as they were
+        assert (got[:, -1] == float("inf")).all()
+        assert torch.equal(got[:, :-1].contiguous().view(torch.int16), clean[:, :-1].contiguous().view(torch.int16))
+    else:
+        assert (got == float("inf")).all()
