@@ -164,13 +164,20 @@ def decode_transposed_hip(weight: torch.Tensor, scale: torch.Tensor) -> torch.Te
     return out
 
 
+def _matrix(tensor: torch.Tensor) -> torch.Tensor:
+    # the two calls that change nothing on a matrix take as long on the host as all checks together
+    if tensor.ndim == 2 and tensor.is_contiguous():
+        return tensor
+    return tensor.reshape(-1, tensor.shape[-1]).contiguous()
+
+
 def _check_weight(weight: torch.Tensor, scale: torch.Tensor) -> None:
     """Every path hands the weight and its scales to a kernel by address: what they must be for that."""
 
     if weight.ndim != 2 or weight.dtype != torch.int8 or not weight.is_contiguous():
         raise RuntimeError("HIP int8 weight must be a contiguous int8 matrix.")
     if scale.dtype != torch.float32 or scale.numel() != weight.shape[0] or not scale.is_contiguous() \
-            or scale.device != weight.device:
+            or scale.get_device() != weight.get_device():
         raise RuntimeError("HIP int8 scale must be contiguous float32 on the weight's device, one a row of the weight.")
 
 
@@ -179,9 +186,10 @@ def _misfit(matrix: torch.Tensor, weight: torch.Tensor, features: int, bias: tor
     """Why the kernels that take the activations by address cannot read them (None when they can):
     they rely on the sizes they are given."""
 
-    if matrix.dtype != torch.bfloat16 or matrix.device != weight.device or matrix.shape[1] != features:
+    if matrix.dtype != torch.bfloat16 or matrix.get_device() != weight.get_device() or matrix.shape[1] != features:
         return f"expected bfloat16 rows of {features} on the weight's device"
-    if bias is not None and (bias.numel() != outputs or bias.shape[-1:] != (outputs,) or bias.device != weight.device):
+    if bias is not None and (bias.numel() != outputs or bias.shape[-1:] != (outputs,)
+                             or bias.get_device() != weight.get_device()):
         return f"expected a bias of {outputs} on the weight's device"
     return None
 
@@ -205,6 +213,11 @@ def _by_address(*operands: torch.Tensor | None) -> bool:
     return True
 
 
+def _autocast_dtype(tensor: torch.Tensor) -> torch.dtype:
+    kind = tensor.device.type
+    return torch.get_autocast_dtype(kind) if torch.is_autocast_enabled(kind) else torch.bfloat16
+
+
 def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: int, backward: bool,
            matrix: torch.Tensor, out: torch.Tensor | None, bias: torch.Tensor | None = None, *,
            misfit: str | None = None) -> str:
@@ -225,8 +238,7 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
     plain = not misfit and _by_address(matrix, out, bias)
     if misfit or not plain and out is None:
         return "library"
-    kind = matrix.device.type
-    if torch.is_autocast_enabled(kind) and torch.get_autocast_dtype(kind) != torch.bfloat16:
+    if torch._C._is_any_autocast_enabled() and _autocast_dtype(matrix) != torch.bfloat16:
         plain = False  # torch's product returns autocast's type, the strips bfloat16
     long_reduction = reduction >= LONG_REDUCTION * width
     # What the strip kernels' and the transposed decode's argument checks refuse and the library path
@@ -299,7 +311,7 @@ def int8_linear_forward(tokens: torch.Tensor, weight: torch.Tensor, scale: torch
 
     lib = _native.load()
     _check_weight(weight, scale)
-    matrix = tokens.reshape(-1, tokens.shape[-1]).contiguous()
+    matrix = _matrix(tokens)
     rows = matrix.shape[0]
     out_features, in_features = weight.shape
     if bias is not None:
@@ -340,7 +352,7 @@ def int8_linear_backward(gradient: torch.Tensor, weight: torch.Tensor, scale: to
 
     lib = _native.load()
     _check_weight(weight, scale)
-    matrix = gradient.reshape(-1, gradient.shape[-1]).to(torch.bfloat16).contiguous()
+    matrix = _matrix(gradient.to(torch.bfloat16))
     rows = matrix.shape[0]
     out_features, in_features = weight.shape
     route = _route(path, rows, weight, out_features, in_features, True, matrix, out,
