@@ -132,11 +132,14 @@ LONG_REDUCTION = 4
 #   rows                  3400      4608      5700      6400      8192      11000     14000     17792
 #   3072 from 3072       73/66     85/74   113/115   118/122   146/133   198/178   229/201   307/258
 #   12288 from 3072    235/206   312/271   422/363   399/350   501/430   704/654   841/749  1103/945
-# Not for reductions under TRANSPOSED_REDUCTION (6200 rows of 3072 from 1040: 65/77), nor for outputs
-# a power of two wide, where the library's kernel for it is erratic (8192 from 3072: 2800 rows
-# 135/197, 4000 rows 169/150, 5700 rows 280/326), nor for long reductions (3072 from 24576: 7800
-# rows 1483/1536, 8192 rows 1044/923, 8600 rows 1409/1487).
-TRANSPOSED_REDUCTION = 2048
+# Not for reductions outside TRANSPOSED_REDUCTION (6200 rows of 3072 from 1040: 65/77; 5550 rows of
+# 5552 from 18384: 1372/1613), nor below STRIP_ROWS_BACKWARD rows, where the decode is most of the call
+# and writes its rows in shorter pieces (1246 rows of 13168 from 3536: 161/224, 14 rows of 8896 from
+# 12112: 113/152), nor for outputs a power of two wide, where the library's kernel for it is erratic
+# (8192 from 3072: 2800 rows 135/197, 4000 rows 169/150, 5700 rows 280/326), nor for long reductions
+# (3072 from 24576: 7800 rows 1483/1536, 8192 rows 1044/923, 8600 rows 1409/1487). Of 125 random calls
+# inside the range 8 are over 4 % slower (24 % at worst), the mean is 5 % faster.
+TRANSPOSED_REDUCTION = (2048, 6144)
 PATHS = ("auto", "fused", "library", "strip", "transposed")
 
 
@@ -255,7 +258,8 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
         return "library"
     if long_reduction and _splits(rows, width, reduction, backward):
         return "fused"
-    if backward and fits and reduction >= TRANSPOSED_REDUCTION and not long_reduction and width & (width - 1):
+    if (backward and fits and rows >= STRIP_ROWS_BACKWARD and not long_reduction and width & (width - 1)
+            and TRANSPOSED_REDUCTION[0] <= reduction <= TRANSPOSED_REDUCTION[1]):
         return "transposed"
     return "library"
 

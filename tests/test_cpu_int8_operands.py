@@ -201,3 +201,17 @@ def test_autocast_to_another_type_keeps_its_result_type(library) -> None:
     with torch.autocast("cpu", dtype=torch.bfloat16):
         assert qk.int8_linear_forward(x, w, s).dtype == torch.bfloat16
     assert library.names == ["mo_int8_strip_forward"]
+
+
+@pytest.mark.parametrize("rows,out_features,in_features,want", [
+    (2559, 6160, 4096 + 16, "library"), (2560, 3088, 6160, "transposed"), (320, 6160, 3088, "library"),
+    (2560, 2032, 12304, "library"), (2560, 2048, 12304, "transposed"), (2560, 6144, 3088, "transposed"),
+    (2560, 6160, 3088, "library"), (2560, 3072, 8192, "library"), (2559, 3072, 3072, "strip"),
+])
+def test_input_gradients_on_the_transposed_weight(rows, out_features, in_features, want) -> None:
+    """Only from the strips' rows on and for reductions it was measured at; reductions that are no
+    multiple of 64 are not the strips' at any rows."""
+
+    weight = torch.empty(out_features, in_features, dtype=torch.int8, device="meta")
+    matrix = torch.empty(16, dtype=torch.bfloat16)
+    assert qk._route("auto", rows, weight, out_features, in_features, True, matrix, None) == want
