@@ -98,8 +98,12 @@ def decode(weight: torch.Tensor, scale: torch.Tensor, dtype: torch.dtype) -> tor
 #    3072 from 24576      58/284/205   108/148/267   148/174/275   220/257/344   287/349/421   404/701/651   611/931/833
 #    12288 from 3072        35/53/54      64/93/72      77/96/90   119/141/153   155/173/160   196/224/197   302/339/313
 # - input gradients below STRIP_ROWS_BACKWARD rows, and below STRIP_LONG_ROWS where the reduction is
-#   at least LONG_REDUCTION times the output width, for which the library's kernel is weak (8192
-#   rows of 3072 from 24576: strip 1038, library 931 on the transposed weight);
+#   at least LONG_REDUCTION times the output width, for which the library's kernel is erratic (3072
+#   from 24576, strip / library: 3569 rows 490/769, 3884 rows 542/525, 4784 rows 643/877, 5350 rows
+#   694/645, 5477 rows 814/1216), unless the fused plan splits such a reduction and the 128 x 256
+#   tiles no longer fit the CUs two at a time (5350 rows are 504, 5589 are 528 and take 831 against
+#   750 of the fused kernels, 6090 rows 874/824; 5589 from 16384 559/514; 45 random calls past 512
+#   tiles: fused 7 % faster on average, 5 % slower at worst);
 # - forwards below STRIP_ROWS rows, and up to STRIP_ROWS_NARROW while their 128 x 256 tiles fill half
 #   a round of the CUs but hardly more than one (past it a second round starts: 3300 rows of 3072 from 8192 take
 #   175, the library 143; under half a round the large tiles split the reduction as well and the
@@ -110,6 +114,7 @@ STRIP_LONG_ROWS_FORWARD = 1280
 STRIP_TILES, STRIP_ROWS_NARROW = (128, 264), 2816
 STRIP_ROWS_BACKWARD = 2560
 STRIP_LONG_ROWS = 6144
+STRIP_LONG_TILES = 512
 # Any other call with at least LIBRARY_ROWS rows, or a weight of at least LIBRARY_WEIGHT elements,
 # decodes the weight once (mo_int8_decode) and runs the library GEMM on it, unless its reduction is
 # at least LONG_REDUCTION times its output width and the fused kernels' launch plan splits that
@@ -267,11 +272,13 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
 def _strips(rows: int, reduction: int, width: int, backward: bool, long_reduction: bool) -> bool:
     """Whether a call runs the strip kernels (see ``STRIP_ROWS``)."""
 
+    tiles = -(-rows // 128) * -(-width // 256)
     if backward:
-        return rows < (STRIP_LONG_ROWS if long_reduction else STRIP_ROWS_BACKWARD)
+        if rows < STRIP_ROWS_BACKWARD or not long_reduction:
+            return rows < STRIP_ROWS_BACKWARD
+        return rows < STRIP_LONG_ROWS and (tiles <= STRIP_LONG_TILES or not _splits(rows, width, reduction, True))
     if long_reduction and rows >= STRIP_LONG_ROWS_FORWARD and _splits(rows, width, reduction, False):
         return False
-    tiles = -(-rows // 128) * -(-width // 256)
     return rows < STRIP_ROWS or (rows <= STRIP_ROWS_NARROW and STRIP_TILES[0] <= tiles <= STRIP_TILES[1])
 
 

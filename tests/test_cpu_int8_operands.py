@@ -215,3 +215,15 @@ def test_input_gradients_on_the_transposed_weight(rows, out_features, in_feature
     weight = torch.empty(out_features, in_features, dtype=torch.int8, device="meta")
     matrix = torch.empty(16, dtype=torch.bfloat16)
     assert qk._route("auto", rows, weight, out_features, in_features, True, matrix, None) == want
+
+
+@pytest.mark.parametrize("rows,width,splits,want", [
+    (5376, 3072, True, "strip"), (5377, 3072, True, "fused"), (5377, 3072, False, "strip"),
+    (6143, 2560, True, "strip"), (2559, 8192, True, "strip"), (2560, 8192, True, "fused"),
+    (6144, 3072, True, "fused"), (6144, 3072, False, "library"),
+])
+def test_long_input_gradients_leave_the_strips_to_a_split_plan(library, monkeypatch, rows, width, splits, want) -> None:
+    monkeypatch.setattr(qk, "_splits", lambda *args: splits)
+    weight = torch.empty(4 * width, width, dtype=torch.int8, device="meta")
+    matrix = torch.empty(16, dtype=torch.bfloat16)
+    assert qk._route("auto", rows, weight, 4 * width, width, True, matrix, None) == want
