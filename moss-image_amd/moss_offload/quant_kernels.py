@@ -27,6 +27,8 @@ fp16 and fp32, which ``auto`` sends to the eager path here.
 
 from __future__ import annotations
 
+import functools
+
 import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad
@@ -86,7 +88,8 @@ def decode(weight: torch.Tensor, scale: torch.Tensor, dtype: torch.dtype) -> tor
 
 # Calls with few rows run the strip kernels (mo_int8_strip_*, reductions of whole steps of 64). The
 # other paths pay for a decode of the whole weight (8 to 40 us), or for a grid of large tiles that
-# does not fill the GPU. Measured on MI355X, us, strip / fused / library:
+# does not fill the GPU. Measured on the 256 CUs of an MI355X (the rows hold for those; a partition
+# keeps the tiles a CU, unmeasured), us, strip / fused / library:
 #   rows                       320           700           1000          1450          2100          2693          4608
 #   forward
 #    3072 from 3072         15/28/31      25/31/32      30/35/36      41/48/46      43/54/49      54/78/55     82/102/71
@@ -111,10 +114,10 @@ def decode(weight: torch.Tensor, scale: torch.Tensor, dtype: torch.dtype) -> tor
 #   plan splits stay there from STRIP_LONG_ROWS_FORWARD rows (1700 rows of 3072 from 12288: 129 / 126).
 STRIP_ROWS = 1536
 STRIP_LONG_ROWS_FORWARD = 1280
-STRIP_TILES, STRIP_ROWS_NARROW = (128, 264), 2816
+STRIP_TILES, STRIP_ROWS_NARROW = (1 / 2, 33 / 32), 2816  # tiles a CU
 STRIP_ROWS_BACKWARD = 2560
 STRIP_LONG_ROWS = 6144
-STRIP_LONG_TILES = 512
+STRIP_LONG_TILES = 2  # a CU
 # Any other call with at least LIBRARY_ROWS rows, or a weight of at least LIBRARY_WEIGHT elements,
 # decodes the weight once (mo_int8_decode) and runs the library GEMM on it, unless its reduction is
 # at least LONG_REDUCTION times its output width and the fused kernels' launch plan splits that
@@ -255,7 +258,7 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
     fits = weight.numel() < 1 << 31 and all(size % 16 == 0 and size <= 1 << 20 for size in weight.shape)
     if (plain and rows and fits and reduction % 64 == 0 and matrix.data_ptr() % 16 == 0
             and (out is None or out.data_ptr() % 16 == 0)
-            and _strips(rows, reduction, width, backward, long_reduction)):
+            and _strips(rows, reduction, width, backward, long_reduction, _cus(matrix.get_device()))):
         return "strip"
     if rows < LIBRARY_ROWS and weight.numel() < LIBRARY_WEIGHT:
         return "fused"
@@ -269,10 +272,17 @@ def _route(path: str, rows: int, weight: torch.Tensor, reduction: int, width: in
     return "library"
 
 
-def _strips(rows: int, reduction: int, width: int, backward: bool, long_reduction: bool) -> bool:
-    """Whether a call runs the strip kernels (see ``STRIP_ROWS``)."""
+@functools.lru_cache(maxsize=None)
+def _cus(index: int) -> int:
+    """CUs of a device (256 of an MI355X, fewer of a partition of it; off a HIP device as many)."""
 
-    tiles = -(-rows // 128) * -(-width // 256)
+    return torch.cuda.get_device_properties(index).multi_processor_count if index >= 0 else 256
+
+
+def _strips(rows: int, reduction: int, width: int, backward: bool, long_reduction: bool, cus: int) -> bool:
+    """Whether a call runs the strip kernels on a device of ``cus`` CUs (see ``STRIP_ROWS``)."""
+
+    tiles = -(-rows // 128) * -(-width // 256) / cus
     if backward:
         if rows < STRIP_ROWS_BACKWARD or not long_reduction:
             return rows < STRIP_ROWS_BACKWARD

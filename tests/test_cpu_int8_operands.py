@@ -227,3 +227,16 @@ def test_long_input_gradients_leave_the_strips_to_a_split_plan(library, monkeypa
     weight = torch.empty(4 * width, width, dtype=torch.int8, device="meta")
     matrix = torch.empty(16, dtype=torch.bfloat16)
     assert qk._route("auto", rows, weight, 4 * width, width, True, matrix, None) == want
+
+
+@pytest.mark.parametrize("cus", [32, 256])
+def test_the_strips_tiles_are_counted_by_cu(monkeypatch, cus) -> None:
+    """Forwards of 1600 rows (13 row tiles of 128) are strips from half a round of the CUs to hardly
+    more than one, long input gradients whose plan splits up to two rounds."""
+
+    monkeypatch.setattr(qk, "_splits", lambda *args: True)
+    for columns in range(1, 30):  # of 256
+        tiles = 13 * columns
+        assert qk._strips(1600, 512, 256 * columns, False, False, cus) == (cus <= 2 * tiles and 32 * tiles <= 33 * cus)
+    for columns in range(1, 30):
+        assert qk._strips(2560, 1 << 20, 256 * columns, True, True, cus) == (20 * columns <= 2 * cus)
