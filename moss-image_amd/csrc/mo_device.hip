@@ -561,14 +561,18 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_link_copy_kernel(c
 
 
 // ------------------------------------------------------------------------------------------
-// Wire coding of a staging segment (format in mo_wire.h): three kernels code a segment into a
-// wire buffer (each tile's exponent model and rANS stream into the working space, with its
-// coded size; a one-workgroup scan of the tile sizes into offsets plus the header and the raw
-// tail; then each tile assembled at its offset), and one kernel decodes it. One wave codes or
-// decodes one tile, four waves a workgroup; the waves share no LDS and never wait for each
-// other. Every store into the wire buffer goes through a buffer resource bounded by the
-// buffer's capacity, and the decoder reads the coded stream through one too, so a stream that
-// arrives damaged cannot make either kernel touch memory outside its buffers.
+// Wire coding of a staging segment (format in mo_wire.h). Three kernels code a segment into a
+// wire buffer: each tile's exponent model and rANS stream into the working space, with its coded
+// size (a wave per tile, four a workgroup, which share no LDS and never wait for each other); a
+// scan of the tile sizes into offsets plus the header and the raw tail (one workgroup, whose waves
+// meet once per 4 096 tiles); then each tile assembled at its offset (a workgroup per tile). Two
+// kernels decode one, a workgroup of one wave per tile: one looks a slot's rank up first, the
+// other its whole entry, for segments whose tiles are all resident with that table.
+// Stores into the wire buffer go through a buffer resource bounded by the buffer's capacity, those
+// of a tile's stream words through one over the 32 KiB that the working space keeps for them: the
+// callers pass at least wire_capacity(raw_bytes), which covers both (mo_wire_encode checks it). The
+// decoder reads the coded stream through a resource too, so a stream that arrives damaged cannot
+// make it touch memory outside its buffers.
 namespace mo {
 constexpr int kWireWaves = kThreads / 64;
 constexpr uint32_t kWireOob = 0x80000000u;  // a buffer offset past every wire buffer: the access is dropped
@@ -628,8 +632,9 @@ __device__ __forceinline__ void wave_lds_fence() {
 // Coder table entry of one exponent of frequency f and cumulative frequency c: {f << 20, less one (a
 // state above it emits a word first); f and 4096 - f as the halves of a word; the float just under
 // 1 / f by which a state is divided; c}. With 1 / f * (1 - 2^-22) rounded, trunc(float(x) * that)
-// is floor(x / f) or one less for every x < f << 20: the quotient is under 2^20, and the three
-// roundings, 2^-24 each, and the 2^-22 together stay between 2^-24 and 2^-21 below it.
+// is floor(x / f) or one less for every x < f << 20: four roundings of at most 2^-24 each (of 1 / f,
+// of it times 1 - 2^-22, of float(x), of their product) keep the product above x / f * (1 - 2^-21),
+// which is less than a half below x / f under 2^20, and (1 - 2^-22)(1 + 2^-24)^4 < 1 keeps it below.
 __device__ __forceinline__ float coder_rcp(uint32_t f) { return (1.0f / (float)f) * (1.0f - 0x1p-22f); }
 }  // namespace mo
 
@@ -646,8 +651,8 @@ __device__ __forceinline__ float coder_rcp(uint32_t f) { return (1.0f / (float)f
 // leave about three lanes an address): three instructions a word where adding once per distinct
 // value of a lane's 8 words took 21. A round divides by a float reciprocal with one correction
 // step, where the multiply-high and the low product take four times the issue of the others each;
-// the entries it needs are read a group ahead of the coding chain. A 113 MB Gaussian segment:
-// 97 us before, 66 now; a 256 KiB segment's whole coding 47 us before, 33 now.
+// the entries it needs are read a group ahead of the coding chain. A 113 MB segment of activations,
+// warm: 92 us before, 64 now (105 and 85 from memory); a 256 KiB segment 45 us before, 28 now.
 extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_wire_sizes_kernel(const char* raw, uint64_t raw_bytes,
                                                                                  char* wire, uint64_t wire_capacity) {
   using namespace mo;
@@ -854,8 +859,8 @@ extern "C" __global__ __launch_bounds__(mo::kWireScanThreads) void mo_wire_scan_
 // bytes, table, final states and stream from the working space). One workgroup a tile: HBM-bound
 // (the raw words once more, the stream, 0.67 of the raw bytes out), so every lane has its 8 loads
 // of raw words in flight before it knows the tile's record, and stores and loads are coalesced
-// runs of a wave. A 113 MB segment: 56 us with one wave a tile and 4-byte stream copies, now 32.5
-// (113 MB of raw words and 19 of stream in, 76 of coded bytes out: 6.4 TB/s).
+// runs of a wave. A 113 MB segment: 56 us with one wave a tile and 4-byte stream copies, now 32.7
+// (113 MB of raw words and 19 of stream in, 76 of coded bytes out: 6.4 TB/s); 58 and 35 from memory.
 extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_wire_encode_kernel(const char* raw, uint64_t raw_bytes,
                                                                                   char* wire, uint64_t wire_capacity) {
   using namespace mo;
@@ -939,8 +944,10 @@ extern "C" __global__ __launch_bounds__(mo::kThreads) void mo_wire_encode_kernel
 // kDirect: the slots' table holds whole entries (16 KiB; 20 KiB a tile, 8 tiles a CU), two LDS reads
 // a round. Otherwise it holds ranks (4 KiB; 8 KiB a tile, 20 tiles a CU), whose entries a third read
 // brings; an entry's parts sit where the multiply, the subtraction and the byte store take them as
-// they are. 113 MB: 67 us with four tiles a workgroup and 26 instructions a round, 53.5 by ranks now;
-// a 256 KiB segment 48 us, 33 by ranks, 29.7 direct.
+// they are. 113 MB: 66 us with four tiles a workgroup and 26 instructions a round, 51 by ranks now; a
+// 256 KiB segment 47 us, 33 by ranks, 30 direct. These are calls back to back, the stream in the
+// cache; from memory every tile also waits for the chain of loads in front of its first round (tile
+// offset, head, then table, states and stream): 80 and 76 us, 51 and 40 by ranks, 37 direct.
 // Reads go through a resource over [wire, wire + wire_bytes), and writes stay inside
 // [raw, raw + raw_bytes) whatever the stream holds: a damaged header is clamped, and table values
 // only index the wave's own LDS arrays.

@@ -356,9 +356,10 @@ int wire_decode(uint64_t wire, uint64_t wire_bytes, uint64_t raw, uint64_t raw_b
   void* r = (void*)raw;
   uint64_t wb = wire_bytes, n = raw_bytes;
   void* params[] = {&w, &wb, &n, &r};
-  // Whole entries a slot while every tile is resident with them (8 a CU: 64 MiB on 256 CUs): 256 KiB
-  // 32.7 us by ranks and 29.7 direct, 16 MiB 37.1 and 34.6, 63 MiB 43.4 and 41.3. One tile more
-  // waits for a whole tile's time: 72 MiB 45.9 by ranks, 69.5 direct.
+  // Whole entries a slot while every tile is resident with them (8 a CU: 64 MiB on 256 CUs). By ranks
+  // and direct, us, back to back and (from memory): 256 KiB 32.6 and 29.7 (40 and 38), 16 MiB 37.1
+  // and 34.5 (47.5 and 45.6), 63 MiB 44.0 and 42.0 (64.8 and 65.5). One tile more waits for a whole
+  // tile's time: 72 MiB 46.4 and 69.7 (68 and 95).
   const hipFunction_t fn = tiles <= m.direct_tiles ? m.wire_decode_direct : m.wire_decode;
   return (int)hipModuleLaunchKernel(fn, tiles ? (uint32_t)tiles : 1, 1, 1, kWireLanes, 1, 1, 0, stream, params,
                                     nullptr);  // a wave per tile

@@ -7,7 +7,7 @@
 // s(1) e(8) m(7), in tiles of up to 32 blocks of 512 words (32 KiB raw). A tile keeps each
 // word's sign and mantissa as one byte and codes the 8-bit exponent fields with interleaved rANS
 // (range asymmetric numeral systems): 64 coder states, state l taking the tile's words
-// l*J .. l*J + J - 1 (J = the tile's words / 64), 32-bit states kept in [2^16, 2^32), 16-bit
+// 64 j + l, j = 0 .. J - 1 (J = the tile's words / 64), 32-bit states kept in [2^16, 2^32), 16-bit
 // renormalisation words, and the tile's exponent frequencies normalised to 4096:
 //   f(e) = floor(count(e) * 4096 / words) for every exponent e present, at least 1, and the
 //   difference of their sum to 4096 added to the most frequent exponent (the smallest on ties).
