@@ -128,10 +128,15 @@ def test_operands_off_the_grid_run_as_on_the_library_path() -> None:
         decoded = quant_kernels.decode(w, scale, torch.bfloat16).double()
         decoded = decoded if backward else decoded.t()
         for matrix, buffer in ((off, None), (a, out)):
-            if backward:
-                got = quant_kernels.int8_linear_backward(matrix, w, scale, torch.Size((rows, width)), out=buffer)
-            else:
-                got = quant_kernels.int8_linear_forward(matrix, w, scale, b, out=buffer)
+            def call(path):
+                if backward:
+                    return quant_kernels.int8_linear_backward(matrix, w, scale, torch.Size((rows, width)), out=buffer,
+                                                              path=path)
+                return quant_kernels.int8_linear_forward(matrix, w, scale, b, out=buffer, path=path)
+
+            named = call("library").clone()
+            got = call("auto")
+            assert torch.equal(got.view(torch.int16), named.view(torch.int16))
             exact = a.double() @ decoded + (0 if backward else b.double())
             _within_accumulation_bound(got, exact, a.double().abs() @ decoded.abs(), a.shape[1])
 
