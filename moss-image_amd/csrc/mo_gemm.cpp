@@ -71,6 +71,10 @@ constexpr Strip kStrips[kStripCount] = {
     {"64x64k4", 64, 64, 4, 1, 6.3, 0.67, 0.67},      // a 3 072-wide output of a few hundred rows
     {"32x64k4", 32, 64, 4, 2, 4.0, 0.49, 1.31},      // fewer rows than that
 };
+// Below 28 steps (reductions under 1792) a split gains nothing on the GPU (112 calls replayed from
+// graphs: 0.87 to 1.20 of the unsplit time, 1.00 on average), and its second launch takes the host
+// 5 us (24 rows of 192 from 1280: 18.6 us split, where the large-tile path takes 14.5).
+constexpr uint32_t kMinStripSplit = 28;
 constexpr double kStripReduce = 1.5, kStripReducePerMb = 0.28;  // the plane sum: fixed, per MB of planes
 
 // Which kernel takes the large-tile rows of a launch plan (mo_int8_set_kernel).
@@ -283,8 +287,8 @@ double strip_cost(const Strip& s, uint32_t rows, uint32_t cols, uint32_t splits,
   return cost;
 }
 
-// The cheapest strip call. Splits: at most 32, of at least 6 steps (64-row tiles of four K groups
-// at least 8, two a group), while the workgroups stay within four and a half rounds of the CUs (more only pay for
+// The cheapest strip call. Splits: at most 32, of at least 6 steps, from reductions of kMinStripSplit
+// steps on, while the workgroups stay within four and a half rounds of the CUs (more only pay for
 // planes). The 64 x 64 tile, one workgroup a CU, only while its grid fits one round: past it the
 // 32-row tile, two a CU, or the 128-row ones were faster at every size measured.
 StripPlan strip_plan(uint32_t rows, uint32_t cols, uint32_t steps, int cus, bool may_split) {
@@ -295,7 +299,8 @@ StripPlan strip_plan(uint32_t rows, uint32_t cols, uint32_t steps, int cus, bool
     const uint64_t tiles = div_up(rows, s.bm) * div_up(cols, s.bn);
     uint32_t tried = 0;
     for (uint32_t want = 1; want <= 32; ++want) {
-      if (want > 1 && (!may_split || steps / want < 6 || 2 * tiles * want > 9ull * cus)) break;
+      if (want > 1 && (!may_split || steps < kMinStripSplit || steps / want < 6 || 2 * tiles * want > 9ull * cus))
+        break;
       const uint32_t per = (steps + want - 1) / want, splits = (steps + per - 1) / per;
       if (splits == tried) continue;
       tried = splits;

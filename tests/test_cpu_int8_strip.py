@@ -76,3 +76,13 @@ def test_route_leaves_the_library_what_the_strips_refuse(backward) -> None:
     assert route(320, odd, grid, None) == route(320, huge, grid, None) == "library"
     # calls of the fused kernels' size stay with them, and are refused there as before
     assert route(320, weight[:3072], off, None) == "fused"
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 64), (24, 192), (294, 128), (700, 6160)])
+def test_short_reductions_are_not_split(rows, cols) -> None:
+    """A split pays for its second launch from 28 steps on, and a tile that is far from filling the
+    CUs is split from there."""
+
+    for steps in range(1, 28):
+        assert qk.strip_plan(rows, cols, 64 * steps, CUS)["splits"] == 1
+    assert (qk.strip_plan(rows, cols, 64 * 28, CUS)["splits"] > 1) == (rows < 700)
