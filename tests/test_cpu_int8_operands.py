@@ -240,3 +240,16 @@ def test_the_strips_tiles_are_counted_by_cu(monkeypatch, cus) -> None:
         assert qk._strips(1600, 512, 256 * columns, False, False, cus) == (cus <= 2 * tiles and 32 * tiles <= 33 * cus)
     for columns in range(1, 30):
         assert qk._strips(2560, 1 << 20, 256 * columns, True, True, cus) == (20 * columns <= 2 * cus)
+
+
+def test_a_named_buffer_ends_no_graph_silently(library) -> None:
+    """With a buffer torch's product refuses operands that want a graph; the smaller weights' kernels
+    write it, as a caller that names one asks for."""
+
+    x, _, w, s = _operands("library")
+    with pytest.raises(RuntimeError, match="out="):
+        qk.int8_linear_forward(x.clone().requires_grad_(True), w, s, out=torch.empty(20, w.shape[0]).bfloat16())
+    assert library.names == []
+    x, _, w, s = _operands("small")
+    qk.int8_linear_forward(x.clone().requires_grad_(True), w, s, out=torch.empty(20, w.shape[0]).bfloat16())
+    assert library.names == ["mo_int8_linear_forward"]
