@@ -14,7 +14,8 @@ three ways in the same process on the same seeds:
 Regime A: every block under non-reentrant checkpointing (the reference default), so the hook
 sees each block's inputs. Regime B: no checkpointing, so the hook sees every activation.
 
-Prints ONE JSON line (stdout). Progress goes to stderr.
+Prints ONE JSON line (stdout) with every leg's step times and rates; the whole record, 30 KB of
+counters, goes to --detail. Progress goes to stderr.
 
 Leg Q: the config-5 int8 weight-only GEMMs on the HIP MFMA kernels against the eager path.
 Leg BR: regime B on the first 16 blocks, where the reference hooks' pinned copies fit the host.
@@ -1448,6 +1449,39 @@ def run(args) -> dict:
     return result
 
 
+# what the printed line keeps of a leg's mode and of the microbench; the rest is in --detail
+BRIEF_LEG = ("s_per_it", "exposed_s", "exposed_s_median", "hidden_fraction", "hidden_fraction_median", "d2h_gbps",
+             "h2d_gbps", "peak_device_bytes", "skipped")
+BRIEF_MICRO = ("s_per_iter", "d2h_gbps", "h2d_gbps", "pack_hbm_gbps", "unpack_hbm_gbps", "bitwise_first", "bitwise_last")
+
+
+def brief(result: dict) -> dict:
+    """The part of the record that the printed line carries: readers that keep only the last 8 KB of
+    the output must still find the line whole."""
+
+    def pick(figures: dict, keys: tuple[str, ...]) -> dict:
+        kept = {k: figures[k] for k in keys if figures.get(k) is not None}
+        return {k: float(f"{v:.5g}") if isinstance(v, float) else v for k, v in kept.items()}
+
+    out = {k: result[k] for k in ("link", "parity") if k in result}
+    out["regimes"] = {name: {mode: pick(figures, BRIEF_LEG) for mode, figures in leg.items() if isinstance(figures, dict)}
+                      for name, leg in result["regimes"].items()}
+    if "micro" in result:
+        out["micro"] = pick(result["micro"], BRIEF_MICRO)
+    if "int8_gemm" in result:
+        out["int8_gemm"] = {k: v for k, v in result["int8_gemm"].items() if k.startswith("block_")}
+    return out
+
+
+def write_detail(path: str, record: dict) -> None:
+    try:
+        os.makedirs(os.path.dirname(path) or ".", exist_ok=True)
+        with open(path, "w") as f:
+            json.dump(record, f, default=float, indent=1)
+    except OSError as e:  # the measurements are printed all the same
+        log(f"whole record not written: {e}")
+
+
 def main() -> int:
     parser = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     parser.add_argument("--gpus", type=int, default=1)
@@ -1536,6 +1570,8 @@ def main() -> int:
     parser.add_argument("--int8-backend", default="auto", choices=("auto", "eager", "hip"),
                         help="backend of config 5's int8 bases (auto = the HIP MFMA kernels when supported)")
     parser.add_argument("--cpu-budget", type=float, default=15.0)
+    parser.add_argument("--detail", default=str(ROOT / "build" / "bench_detail.json"),
+                        help="file for the whole record, every counter of every leg ('': not written)")
     args = parser.parse_args()
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
@@ -1626,8 +1662,10 @@ def main() -> int:
         "roofline": pack_bound,
         "int8_gemm_roofline": result.get("int8_gemm", {}).get("roofline"),
         "cpu_baseline": cpu,
-        "detail": result,
+        "detail": brief(result),
     }
+    if args.detail:
+        write_detail(args.detail, {**line, "detail": result})
     print(json.dumps(line, default=float), flush=True)
     return 0
 
