@@ -889,7 +889,7 @@ def int8_gemm_leg(device, iters: int = 20, warmup: int = 3, rounds: int = 3) -> 
         "long_reduction_ratio": qk.LONG_REDUCTION,
         "timing": f"median of {rounds} interleaved rounds of {iters} calls per path",
         "roofline": {"bound": "mfma",
-                     "kernels": ("auto dispatch at these rows: mo_int8_ws_{fwd,kscale}_split + mo_int8_split_reduce "
+                     "kernels": ("auto dispatch at these rows: mo_int8_ws_{fwd,kscale} (+ _split, mo_int8_split_reduce) "
                                  f"where the reduction is >= {qk.LONG_REDUCTION}x the output width and the plan splits "
                                  "it, else the library GEMM on the weight as mo_int8_decode_kernel, or for input "
                                  f"gradients from {qk.TRANSPOSED_REDUCTION[0]} to {qk.TRANSPOSED_REDUCTION[1]} features "
